@@ -151,8 +151,8 @@ struct Publish {
 // kStageMax of them are loaded into LDS once per sweep (coalesced) and the
 // block's fluid lists are 16-bit indices into the set; sets up to kStageCap
 // keep the 16-bit lists and read the particles through the set's global ids;
-// larger ones (sparse splashes, more than kAdjMax / 27 own cells, the
-// unsorted search) use 32-bit global lists (stage_n = kUnstaged).
+// larger ones, blocks spread over too many cells for the search's tables and
+// the unsorted search use 32-bit global lists (stage_n = kUnstaged).
 // LDS-staged particles per block.  A set read through its global ids instead
 // costs about 1.5x per sweep, more than the occupancy a smaller stage would
 // win, so the cap holds nearly every set.  256-particle blocks: 2048 (C2 sets:
@@ -195,7 +195,6 @@ constexpr uint32_t kStageMaxX = DFSPH_X_STAGE;
 constexpr uint32_t kStageCap = 4096;       // largest set with 16-bit lists
 constexpr uint32_t kUnstaged = 0xffffffffu;
 constexpr uint32_t kSetNoLds = 0x80000000u;  // stage_n flag: 16-bit lists, set not in LDS
-constexpr uint32_t kAdjMax = 2048;         // 27 x unique own cells per block
 constexpr uint32_t kKeyInvalid = 0xffffffffu;
 constexpr uint32_t kGroup16 = 8;           // entries per 16-byte group
 constexpr uint32_t kGroup32 = 4;
@@ -526,6 +525,31 @@ __device__ __forceinline__ void for_each_adjacent_cell(const SimConst& c, int cx
     }
 }
 
+// The same 27 cells as ranges of the cell table cs, row by row: the keys and
+// table reads of a row's three cells are in flight together (a cell at a
+// time would wait for each).
+template <class F>
+__device__ __forceinline__ void for_each_adjacent_range(const SimConst& c, int cx, int cy, int cz,
+                                                        const uint32_t* __restrict__ cs, F&& f)
+{
+#pragma unroll 1
+    for (int r = 0; r < 9; ++r) {
+        const int y = cy + r / 3 - 1, z = cz + r % 3 - 1;
+        if (y < 0 || y >= c.dim[1] || z < 0 || z >= c.dim[2]) continue;
+        uint32_t s[3], e[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int x = cx + k - 1;
+            const bool in = x >= 0 && x < c.dim[0];
+            const uint32_t key = cell_key(c, in ? x : cx, y, z);
+            s[k] = cs[key];
+            e[k] = in ? cs[key + 1] : s[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) f(s[k], e[k]);
+    }
+}
+
 // Neighbor loops with memory-level parallelism: a batch of 8 list entries is
 // one 16-byte load (16-bit lists) or two (32-bit lists) per lane, then the 8
 // neighbors' gathers can all be in flight before the first one is used.  The
@@ -772,15 +796,25 @@ __device__ __forceinline__ uint32_t wave_sum_u(uint32_t v)
     return v;
 }
 
+// Cross-lane steps as DPP operands of the vector ALU: row_shr 1, 2, 4, 8 inside
+// the rows of 16 lanes, then row_bcast 15 and 31 across them, so that lane k
+// holds op over lanes 0..k (a lane's missing source counts as `ident`).  All 64
+// lanes must be active.  A shuffle would be an LDS instruction per step.
+template <class Op>
+__device__ __forceinline__ uint32_t wave_prefix_dpp(uint32_t v, uint32_t ident, Op&& op)
+{
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)ident, (int)v, 0x111, 0xf, 0xf, false));
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)ident, (int)v, 0x112, 0xf, 0xf, false));
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)ident, (int)v, 0x114, 0xf, 0xf, false));
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)ident, (int)v, 0x118, 0xf, 0xf, false));
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)ident, (int)v, 0x142, 0xa, 0xf, false));
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)ident, (int)v, 0x143, 0xc, 0xf, false));
+    return v;
+}
+
 __device__ __forceinline__ uint32_t wave_incl_scan_u(uint32_t v)
 {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t w = __shfl_up(v, o, 64);
-        if (lane >= o) v += w;
-    }
-    return v;
+    return wave_prefix_dpp(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 // Block-wide exclusive scan (kBlock threads); returns the block total to

@@ -302,28 +302,30 @@ __global__ void k_gather_f4(uint32_t n, const uint32_t* perm, const float4* in, 
 
 // Appends list entries to a particle's blocked-interleaved list: entries
 // shift into a 16-byte register group from the top (a funnel shift per word)
-// and each full group is one store.
+// and each full group is one store at the running group pointer.
 struct ListWriter16 {
-    uint4* out;                    // group 0 of this particle
-    uint32_t cap;
+    uint4* out;                    // the particle's next group
+    uint32_t cap;                  // groups are cap apart
+    uint32_t n = 0;                // entries pushed
     uint32_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
-    __device__ void shift_in(uint32_t v)
+    __device__ __forceinline__ void shift_in(uint32_t v)
     {
         w0 = __builtin_amdgcn_alignbit(w1, w0, 16);
         w1 = __builtin_amdgcn_alignbit(w2, w1, 16);
         w2 = __builtin_amdgcn_alignbit(w3, w2, 16);
         w3 = __builtin_amdgcn_alignbit(v, w3, 16);
     }
-    __device__ void push(uint32_t n, uint32_t v)      // v = entry n (16 bits)
+    __device__ __forceinline__ void push(uint32_t v)  // 16 bits
     {
         shift_in(v);
-        if ((n & 7u) == 7u) out[(size_t)(n >> 3) * cap] = make_uint4(w0, w1, w2, w3);
+        ++n;
+        if ((n & 7u) == 0u) { *out = make_uint4(w0, w1, w2, w3); out += cap; }
     }
-    __device__ void finish(uint32_t n)                // n entries pushed in total
+    __device__ __forceinline__ void finish()
     {
         if (n & 7u) {
             for (uint32_t k = n & 7u; k < 8u; ++k) shift_in(0u);
-            out[(size_t)(n >> 3) * cap] = make_uint4(w0, w1, w2, w3);
+            *out = make_uint4(w0, w1, w2, w3);
         }
     }
 };
@@ -331,63 +333,123 @@ struct ListWriter16 {
 struct ListWriter32 {
     uint4* out;
     uint32_t cap;
+    uint32_t n = 0;
     uint32_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
-    __device__ void shift_in(uint32_t v)
+    __device__ __forceinline__ void shift_in(uint32_t v)
     {
         w0 = w1;
         w1 = w2;
         w2 = w3;
         w3 = v;
     }
-    __device__ void push(uint32_t n, uint32_t v)
+    __device__ __forceinline__ void push(uint32_t v)
     {
         shift_in(v);
-        if ((n & 3u) == 3u) out[(size_t)(n >> 2) * cap] = make_uint4(w0, w1, w2, w3);
+        ++n;
+        if ((n & 3u) == 0u) { *out = make_uint4(w0, w1, w2, w3); out += cap; }
     }
-    __device__ void finish(uint32_t n)
+    __device__ __forceinline__ void finish()
     {
         if (n & 3u) {
             for (uint32_t k = n & 3u; k < 4u; ++k) shift_in(0u);
-            out[(size_t)(n >> 2) * cap] = make_uint4(w0, w1, w2, w3);
+            *out = make_uint4(w0, w1, w2, w3);
         }
     }
 };
 
 // Neighbor-search tables.  A block's set cells are the grid cells within one
-// cell of its own cells; they are indexed through a dense table over the
-// bounding box of those cells, x fastest, then z, then y, so the set lists
-// them in (y, z, x) order and the three cells x-1..x+1 of any row (y, z) are
-// consecutive: one contiguous range of the set per row.
-// LDS of the search with 512-particle blocks: 2672 staged positions and 512
-// set cells take 52 KB, three blocks per CU.  The search is bound by the
-// latency of its per-block phases (set construction, staging, candidate
-// tests between barriers), so the third block gains more than the larger
-// stage of two blocks per CU would (C4: 0.62 against 0.76 ms per search);
-// larger sets search through global memory.
+// cell of its own cells, in (y, z, x) order.  They are collected as one 64-bit
+// mask of x positions per row (y, z) of their bounding box; a cell's number is
+// its row's first number plus the marked cells before it in the row, so the
+// three cells x-1..x+1 of any row are consecutive: one contiguous range of
+// the set per row.
+// LDS of the search with 512-particle blocks: 2688 staged positions (12 B each)
+// and 512 set cells take 40 KB (sets above that search through global
+// memory).  Sparse blocks (spray) have many cells and few particles: tables of
+// up to kBigCells cells take the upper half of the stage when the set fits the
+// lower half.
 #ifndef DFSPH_NBR_STAGE
-#define DFSPH_NBR_STAGE (DFSPH_BLOCK == 512 ? 2672 : 2048)
+#define DFSPH_NBR_STAGE (DFSPH_BLOCK == 512 ? 2688 : 2048)
 #endif
 constexpr uint32_t kNbrStage = DFSPH_NBR_STAGE;   // set positions staged in LDS by the search
-constexpr uint32_t kDense = 8192;          // bounding-box cells of a tabled set
+static_assert(kNbrStage % 16 == 0, "halves, and rows in whole words");
+constexpr uint32_t kHalfStage = kNbrStage / 2;
+constexpr uint32_t kSetRows = kHalfStage * 3 / 4; // rows (y, z) of a tabled set's bounding box
 #ifndef DFSPH_SET_CELLS
 #define DFSPH_SET_CELLS (DFSPH_BLOCK == 512 ? 512 : 384)
 #endif
-constexpr uint32_t kSetCells = DFSPH_SET_CELLS;   // set cells of a tabled set
+constexpr uint32_t kSetCells = DFSPH_SET_CELLS;   // set cells with a full stage
+constexpr uint32_t kBigCells = kHalfStage - 1;    // set cells with half a stage
 constexpr uint32_t kNoRow = 0xffffffffu;
 constexpr int kIntMax = 0x7fffffff;
 
 __device__ __forceinline__ int wave_min_i(int v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-    return v;
+    auto op = [](uint32_t a, uint32_t b) { return (uint32_t)min((int)a, (int)b); };
+    return __builtin_amdgcn_readlane((int)wave_prefix_dpp((uint32_t)v, (uint32_t)kIntMax, op), 63);
 }
 
 __device__ __forceinline__ int wave_max_i(int v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-    return v;
+    auto op = [](uint32_t a, uint32_t b) { return (uint32_t)max((int)a, (int)b); };
+    return __builtin_amdgcn_readlane((int)wave_prefix_dpp((uint32_t)v, (uint32_t)(-kIntMax - 1), op), 63);
+}
+
+__device__ __forceinline__ uint32_t wave_total_u(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan_u(v), 63);
+}
+
+// m = 2 m + (d2 < limit): the compare's carry joins the shift, two vector
+// instructions per candidate (false for a NaN distance).
+__device__ __forceinline__ uint32_t shift_in_less(uint32_t m, float d2, float limit)
+{
+    asm("v_cmp_gt_f32_e32 vcc, %2, %1\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(d2), "s"(limit) : "vcc");
+    return m;
+}
+
+// Staged positions of a set, two at a time: x0 x1 y0 y1 z0 z1.  Four positions
+// are 48 consecutive bytes, three reads at one address.
+struct PosStage {
+    float d[3 * kNbrStage + 12];   // the candidate tests read up to three positions past a range
+    __device__ __forceinline__ void put(uint32_t k, const float4& p)
+    {
+        float* q = d + 6u * (k >> 1) + (k & 1u);
+        q[0] = p.x; q[2] = p.y; q[4] = p.z;
+    }
+};
+
+// Which of the staged positions [l0, min(l0 + 32, e)) lie within the support of
+// p: bit k for l0 + k.  l0 is even; each step tests four positions, 8 vector
+// instructions a candidate.  The last step may test up to three positions past
+// e, whose bits are cleared.
+__device__ __forceinline__ uint32_t near_mask(const PosStage& st, const float4& p, float hk2, uint32_t l0, uint32_t e)
+{
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(8)));
+    const uint32_t cnt = min(e - l0, 32u);
+    uint32_t m = 0, t = 3u * l0;                         // in words
+    const uint32_t end = t + 3u * cnt;
+#pragma unroll 1
+    do {
+        const f4 a = *reinterpret_cast<const f4*>(st.d + t), b = *reinterpret_cast<const f4*>(st.d + t + 4),
+                 c = *reinterpret_cast<const f4*>(st.d + t + 8);
+        m = shift_in_less(m, dist2(p.x - a[0], p.y - a[2], p.z - b[0]), hk2);
+        m = shift_in_less(m, dist2(p.x - a[1], p.y - a[3], p.z - b[1]), hk2);
+        m = shift_in_less(m, dist2(p.x - b[2], p.y - c[0], p.z - c[2]), hk2);
+        m = shift_in_less(m, dist2(p.x - b[3], p.y - c[1], p.z - c[3]), hk2);
+        t += 12u;
+    } while (t < end);
+    // (cnt + 3) / 4 steps made, the first candidate in the highest of their bits
+    m = __builtin_bitreverse32(m) >> ((32u - cnt) & ~3u);
+    return cnt < 32u ? m & ((1u << cnt) - 1u) : m;
+}
+
+// the lowest `count` set bits of m (count < popc(m))
+__device__ __forceinline__ uint32_t lowest_bits(uint32_t m, uint32_t count)
+{
+    uint32_t r = 0;
+    for (; count > 0u; --count) { r |= m & (0u - m); m &= m - 1u; }
+    return r;
 }
 
 // DFSPH_neighborsSearch_kernel<true> (DFSPH_core_cuda.cu:2219-2531,
@@ -398,16 +460,24 @@ __device__ __forceinline__ int wave_max_i(int v)
 // then x) and each cell's particles in index order, in every list form.
 //
 // Each block also builds its neighbor set: the set cells are marked in the
-// dense bounding-box table, numbered by a block scan, and get their fluid
-// ranges, set offsets and boundary ranges.  Every lane then keeps its 9 rows
-// as (first, last) set cells in registers.  Sets up to kNbrStage have their
-// positions staged in LDS for the candidate tests (over the table, which is
-// dead by then); sets up to kStageCap store 16-bit lists; larger ones, blocks
-// whose tables do not fit, and the INDIRECT search (fluid not reordered, the
-// grid indexes it through perm: the need_sort == false path) store 32-bit
-// global lists.
+// row masks, numbered by a block scan over the rows, and get their fluid
+// ranges, set offsets and boundary ranges, one thread per cell.  Every lane then
+// keeps its 9 rows as (first, last) set cells in registers.  Sets up to
+// kNbrStage have their positions staged in LDS for the candidate tests (over
+// the masks, which are dead by then); sets up to kStageCap store 16-bit lists;
+// larger ones, blocks whose tables do not fit, and the INDIRECT search (fluid
+// not reordered, the grid indexes it through perm: the need_sort == false
+// path) store 32-bit global lists.
+//
+// What bounds it: vector instructions (2.7e8 a search of 4.19 M particles, the
+// rate of all SIMDs), over half of them in near_mask's loop and a quarter in
+// the list writers, whose loops run for the wave's longest lane.  64 VGPRs and
+// 40 KB keep four blocks per CU.  Against the version with a dense cell table,
+// binary searches for the stage and 16-byte position records: 597 -> 416 us
+// (4.19 M particles, spacing 2r), one block's walls 15 -> 8 us, and blocks of
+// spray have tables (1 M dam break, 40 steps: 11 -> 5 blocks without).
 template <bool INDIRECT>
-__global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* __restrict__ pos,
+__global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbors(SimConst c, const float4* __restrict__ pos,
                                                       const uint32_t* __restrict__ cs_f,
                                                       const uint32_t* __restrict__ perm,
                                                       const float4* __restrict__ bpos,
@@ -417,19 +487,21 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* 
                                                       uint32_t* __restrict__ stage_n, uint32_t* __restrict__ stg,
                                                       Restrict rs, uint4* __restrict__ part)
 {
-    // the dense table shares one area with the staged positions
-    __shared__ __align__(16) unsigned char s_raw[kNbrStage * sizeof(float4)];
-    __shared__ uint32_t s_off[kSetCells + 1];  // set offsets of the set cells
-    __shared__ uint32_t s_src[kSetCells];      // first fluid index of each set cell
-    __shared__ uint32_t s_bs[kSetCells];       // boundary range of each set cell
-    __shared__ uint32_t s_be[kSetCells];
-    __shared__ uint32_t s_boff[kSetCells + 1]; // boundary set offsets of the set cells
+    // The tables under construction lie in the first half of the staged
+    // positions and are dead once those are loaded.
+    __shared__ __align__(16) PosStage st;
+    unsigned long long* s_mask = reinterpret_cast<unsigned long long*>(st.d);   // x positions of the row's set cells
+    uint32_t* s_place = reinterpret_cast<uint32_t*>(s_mask + kSetRows);   // box place of a set cell: x | z << 6 | y << 16
+    uint16_t* s_first = reinterpret_cast<uint16_t*>(s_place + kBigCells); // number of the row's first set cell
+    static_assert(kSetRows * 10 + kBigCells * 4 <= kHalfStage * 12, "tables under construction exceed half the stage");
+    // four words per set cell (one more for the offsets): set offset of its fluid
+    // particles and what to add for their indices, the same for its boundary ones
+    __shared__ uint32_t s_tab[4 * kSetCells + 2];
+    static_assert(4 * kSetCells + 2 > kBigCells, "the boundary offsets of a large table lie in s_tab");
+    uint32_t *s_off = s_tab, *s_src = s_tab + kSetCells + 1, *s_boff = s_src + kSetCells, *s_bs = s_boff + kSetCells + 1;
     constexpr int NW = kBlock / 64;
     __shared__ int s_w[6 * NW];
-    static_assert(kDense * sizeof(uint16_t) <= sizeof(s_raw), "dense table exceeds the stage");
-    static_assert((kStageCap - 1) * 16 <= 0xffffu && kSetCells < 0xffffu, "16-bit byte offsets / cell ids");
-    uint16_t* s_dense = reinterpret_cast<uint16_t*>(s_raw);
-    float4* s_pos = reinterpret_cast<float4*>(s_raw);
+    static_assert((kStageCap - 1) * 16 <= 0xffffu && kBigCells < 0xffffu, "16-bit byte offsets / cell ids");
     uint32_t* s_wu = reinterpret_cast<uint32_t*>(s_w);
 
     const uint32_t b = xcd_block();
@@ -459,6 +531,7 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* 
             s_w[w] = lo_x; s_w[NW + w] = lo_y; s_w[2 * NW + w] = lo_z;
             s_w[3 * NW + w] = hi_x; s_w[4 * NW + w] = hi_y; s_w[5 * NW + w] = hi_z;
         }
+        for (uint32_t k = threadIdx.x; k < kSetRows; k += kBlock) s_mask[k] = 0ull;
         __syncthreads();
         int lo[3] = {kIntMax, kIntMax, kIntMax}, hi[3] = {-1, -1, -1};
 #pragma unroll
@@ -469,93 +542,113 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* 
                 hi[a] = max(hi[a], s_w[NW * (3 + a) + k]);
             }
         }
-        __syncthreads();                        // s_w is reused by the scans
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            lo[a] = max(lo[a] - 1, 0);
-            hi[a] = min(hi[a] + 1, c.dim[a] - 1);
+            lo[a] = max(__builtin_amdgcn_readfirstlane(lo[a]) - 1, 0);
+            hi[a] = min(__builtin_amdgcn_readfirstlane(hi[a]) + 1, c.dim[a] - 1);
         }
-        const uint32_t W = (uint32_t)(hi[0] - lo[0] + 1), D = (uint32_t)(hi[2] - lo[2] + 1);
-        const uint32_t V = W * D * (uint32_t)(hi[1] - lo[1] + 1);
-        if (V <= kDense) {
-            for (uint32_t k = threadIdx.x; k < V; k += kBlock) s_dense[k] = 0;
-            __syncthreads();
+        const uint32_t W = (uint32_t)(hi[0] - lo[0] + 1), D = (uint32_t)(hi[2] - lo[2] + 1), H = (uint32_t)(hi[1] - lo[1] + 1);
+        if (W <= 64u && D <= kSetRows && H <= kSetRows && D * H <= kSetRows) {
+            const uint32_t R = D * H;
             const int xl = max(cx - 1, 0), xh = min(cx + 1, c.dim[0] - 1);
-            const uint32_t key = act ? cell_key(c, cx, cy, cz) : kKeyInvalid;
-            const bool first = act && ((threadIdx.x & 63) == 0 || __shfl_up(key, 1, 64) != key);
-            if (first) {                        // mark the 27 cells (one lane per run of a cell in a wave)
-                for (int dy = -1; dy <= 1; ++dy) {
-                    const int y = cy + dy;
-                    if (y < 0 || y >= c.dim[1]) continue;
-                    for (int dz = -1; dz <= 1; ++dz) {
-                        const int z = cz + dz;
-                        if (z < 0 || z >= c.dim[2]) continue;
-                        const uint32_t base = W * ((uint32_t)(z - lo[2]) + D * (uint32_t)(y - lo[1])) - lo[0];
-                        for (int x = xl; x <= xh; ++x) s_dense[base + x] = 1;
-                    }
+            const uint32_t bx = (uint32_t)(xl - lo[0]);                            // first x of my rows, in the box
+            const uint32_t nx = (uint32_t)(xh - xl);
+            const uint32_t own = (uint32_t)(cz - lo[2]) + D * (uint32_t)(cy - lo[1]);
+            // mark the 27 cells, one lane per run of a cell in a wave
+            const uint32_t lin = act ? (uint32_t)(cx - lo[0]) + W * own : kKeyInvalid;
+            const uint32_t prev = (uint32_t)__builtin_amdgcn_update_dpp((int)kKeyInvalid, (int)lin, 0x138, 0xf, 0xf, false);
+            if (act && ((threadIdx.x & 63) == 0 || prev != lin)) {
+                const unsigned long long bits = ((2ull << nx) - 1ull) << bx;
+#pragma unroll
+                for (int r = 0; r < 9; ++r) {
+                    const int y = cy + r / 3 - 1, z = cz + r % 3 - 1;
+                    if (y >= 0 && y < c.dim[1] && z >= 0 && z < c.dim[2])
+                        atomicOr(&s_mask[own + (uint32_t)(r % 3 - 1) + D * (uint32_t)(r / 3 - 1)], bits);
                 }
             }
-            __syncthreads();
-            // number the marked cells in table order; thread t owns entries [tE, tE + E)
-            const uint32_t E = (V + kBlock - 1) / kBlock;
-            const uint32_t k0 = threadIdx.x * E, k1 = min(k0 + E, V);
+            __syncthreads();                    // also: s_w is reused by the scans
+            // number the marked cells row by row; thread t owns rows [tE, tE + E)
+            const uint32_t E = (R + kBlock - 1) / kBlock;
+            const uint32_t k0 = threadIdx.x * E, k1 = min(k0 + E, R);
             uint32_t occ = 0;
-            for (uint32_t k = k0; k < k1; ++k) occ += s_dense[k];
+            for (uint32_t k = k0; k < k1; ++k) occ += (uint32_t)__popcll(s_mask[k]);
             uint32_t ubase = 0;
-            U = block_excl_scan_u(occ, &ubase, s_wu);
-            tabled = U <= kSetCells;
+            U = (uint32_t)__builtin_amdgcn_readfirstlane((int)block_excl_scan_u(occ, &ubase, s_wu));
+            const bool big = U > kSetCells;
+            tabled = U <= kBigCells;
+            if (big) {
+                s_off = reinterpret_cast<uint32_t*>(st.d + 3 * kHalfStage);
+                s_src = s_off + kHalfStage;
+                s_bs = s_src + kHalfStage;
+                s_boff = s_tab;
+            }
             if (tabled) {
                 for (uint32_t k = k0; k < k1; ++k) {
-                    if (s_dense[k]) {
-                        const uint32_t u = ubase++;
-                        const uint32_t t = k / W;
-                        const uint32_t key = cell_key(c, lo[0] + (int)(k - t * W), lo[1] + (int)(t / D),
-                                                      lo[2] + (int)(t % D));
-                        const uint32_t a = cs_f[key];
-                        s_src[u] = a;
-                        s_off[u] = cs_f[key + 1] - a;
-                        s_bs[u] = cs_b[key];
-                        s_be[u] = cs_b[key + 1];
-                        s_dense[k] = (uint16_t)u;
+                    const uint32_t y = k / D, at = ((k - y * D) << 6) | (y << 16);
+                    s_first[k] = (uint16_t)ubase;
+                    for (unsigned long long m = s_mask[k]; m != 0ull; m &= m - 1ull)
+                        s_place[ubase++] = at | (uint32_t)(__ffsll((long long)m) - 1);
+                }
+                __syncthreads();
+                // fluid and boundary ranges of the set cells, thread t's being [tC, tC + C)
+                constexpr uint32_t CMAX = (kBigCells + kBlock - 1) / kBlock;
+                const uint32_t C = U <= (uint32_t)kBlock ? 1u : CMAX;
+                uint32_t cf[CMAX], cb[CMAX], f0s[CMAX], b0s[CMAX], fsum = 0, bsum = 0;
+#pragma unroll
+                for (uint32_t k = 0; k < CMAX; ++k) {
+                    const uint32_t u = threadIdx.x * C + k;
+                    cf[k] = cb[k] = f0s[k] = b0s[k] = 0u;
+                    if (k < C && u < U) {
+                        const uint32_t at = s_place[u];
+                        const uint32_t key = cell_key(c, lo[0] + (int)(at & 63u), lo[1] + (int)(at >> 16),
+                                                      lo[2] + (int)((at >> 6) & 1023u));
+                        const uint32_t f0 = cs_f[key], f1 = cs_f[key + 1], b0 = cs_b[key], b1 = cs_b[key + 1];
+                        f0s[k] = f0;
+                        b0s[k] = b0;
+                        cf[k] = f1 - f0;
+                        cb[k] = b1 - b0;
                     }
+                    fsum += cf[k];
+                    bsum += cb[k];
                 }
-            }
-            __syncthreads();
-            if (tabled) {
-                // fluid counts of the set cells -> set offsets
-                const uint32_t E2 = (U + kBlock - 1) / kBlock;
-                const uint32_t u0 = threadIdx.x * E2, u1 = min(u0 + E2, U);
-                uint32_t sum = 0;
-                for (uint32_t u = u0; u < u1; ++u) sum += s_off[u];
-                uint32_t off = 0;
-                const uint32_t tot = block_excl_scan_u(sum, &off, s_wu);
-                for (uint32_t u = u0; u < u1; ++u) {
-                    const uint32_t cu = s_off[u];
-                    s_off[u] = off;
-                    off += cu;
+                // both exclusive scans between one pair of barriers
+                const uint32_t fi = wave_incl_scan_u(fsum), bi = wave_incl_scan_u(bsum);
+                if ((threadIdx.x & 63) == 63) { s_wu[w] = fi; s_wu[NW + w] = bi; }
+                __syncthreads();
+                uint32_t foff = fi - fsum, boff = bi - bsum, tot = 0;
+#pragma unroll
+                for (int k = 0; k < NW; ++k) {
+                    foff += k < w ? s_wu[k] : 0u;
+                    boff += k < w ? s_wu[NW + k] : 0u;
+                    tot += s_wu[k];
+                    Sb += s_wu[NW + k];
                 }
-                if (threadIdx.x == 0) s_off[U] = tot;
+                tot = (uint32_t)__builtin_amdgcn_readfirstlane((int)tot);
+                Sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)Sb);
+#pragma unroll
+                for (uint32_t k = 0; k < CMAX; ++k) {
+                    const uint32_t u = threadIdx.x * C + k;
+                    if (k < C && u < U) {
+                        s_off[u] = foff;
+                        s_boff[u] = boff;
+                        s_src[u] = f0s[k] - foff;
+                        s_bs[u] = b0s[k] - boff;
+                    }
+                    foff += cf[k];
+                    boff += cb[k];
+                }
+                if (threadIdx.x == 0) { s_off[U] = tot; s_boff[U] = Sb; }
                 S = tot <= c.stage_cap ? tot : kUnstaged;
-                // boundary counts -> boundary set offsets (the set's boundary
-                // particles follow its fluid ones when both fit in the stage)
-                uint32_t bsum = 0;
-                for (uint32_t u = u0; u < u1; ++u) bsum += s_be[u] - s_bs[u];
-                uint32_t boff = 0;
-                Sb = block_excl_scan_u(bsum, &boff, s_wu);
-                for (uint32_t u = u0; u < u1; ++u) {
-                    s_boff[u] = boff;
-                    boff += s_be[u] - s_bs[u];
-                }
-                if (threadIdx.x == 0) s_boff[U] = Sb;
                 // each lane's rows (dy, dz) as (first, last) set cell of x-1..x+1
                 if (act) {
-                    uown = s_dense[W * ((uint32_t)(cz - lo[2]) + D * (uint32_t)(cy - lo[1])) + (uint32_t)(cx - lo[0])];
 #pragma unroll
                     for (int r = 0; r < 9; ++r) {
                         const int y = cy + r / 3 - 1, z = cz + r % 3 - 1;
                         if (y >= 0 && y < c.dim[1] && z >= 0 && z < c.dim[2]) {
-                            const uint32_t base = W * ((uint32_t)(z - lo[2]) + D * (uint32_t)(y - lo[1])) - lo[0];
-                            row[r] = (uint32_t)s_dense[base + xl] | ((uint32_t)s_dense[base + xh] << 16);
+                            const uint32_t k = own + (uint32_t)(r % 3 - 1) + D * (uint32_t)(r / 3 - 1);
+                            const uint32_t u = s_first[k] + (uint32_t)__popcll(s_mask[k] & ((1ull << bx) - 1ull));
+                            row[r] = u | ((u + nx) << 16);
+                            if (r == 4) uown = u + (uint32_t)(cx - xl);
                         }
                     }
                 }
@@ -563,31 +656,23 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* 
             }
         }
     }
-    const bool lds_search = S <= kNbrStage && c.stage_lds > 0u;
-    const bool lds_bnd = lds_search && S + Sb <= kNbrStage;   // boundary staged at [S, S + Sb)
+    const uint32_t room = U <= kSetCells ? kNbrStage : kHalfStage;
+    const bool lds_search = S <= room && c.stage_lds > 0u;
+    const bool lds_bnd = lds_search && S + Sb <= room;        // boundary staged at [S, S + Sb)
     if (threadIdx.x == 0) stage_n[b] = S == kUnstaged || S <= c.stage_lds ? S : (S | kSetNoLds);
     if (S != kUnstaged) {
+        // eight lanes per set cell: its particles' ids and positions to their set places
         uint32_t* g_out = stg + (size_t)b * kStageCap;
-        for (uint32_t k = threadIdx.x; k < S; k += kBlock) {
-            uint32_t lo = 0, hi = U;            // the set cell holding set index k
-            while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (s_off[mid] <= k) lo = mid; else hi = mid;
+        const uint32_t sub = threadIdx.x & 7u;
+        for (uint32_t u = threadIdx.x >> 3; u < U; u += kBlock / 8) {
+            const uint32_t off = s_off[u], e = s_off[u + 1u], g0 = s_src[u];
+            for (uint32_t k = off + sub; k < e; k += 8u) {
+                if (lds_search) st.put(k, pos[g0 + k]);
+                g_out[k] = g0 + k;
             }
-            const uint32_t g = s_src[lo] + (k - s_off[lo]);
-            if (lds_search) s_pos[k] = pos[g];
-            g_out[k] = g;
-        }
-        if (lds_bnd) {
-            for (uint32_t k = threadIdx.x; k < Sb; k += kBlock) {
-                uint32_t lo = 0, hi = U;        // the set cell holding boundary set index k
-                while (hi - lo > 1) {
-                    const uint32_t mid = (lo + hi) >> 1;
-                    if (s_boff[mid] <= k) lo = mid; else hi = mid;
-                }
-                const uint32_t j = s_bs[lo] + (k - s_boff[lo]);
-                const float4 q = bpos[j];
-                s_pos[S + k] = make_float4(q.x, q.y, q.z, __uint_as_float(j));   // w: the global boundary id
+            if (lds_bnd) {
+                const uint32_t boff = s_boff[u], be = s_boff[u + 1u], j0 = s_bs[u];
+                for (uint32_t k = boff + sub; k < be; k += 8u) st.put(S + k, bpos[j0 + k]);
             }
         }
         __syncthreads();
@@ -597,60 +682,47 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* 
     if (act && is_source(rs, i)) {
         const uint32_t maxn = c.max_nbr, cap = c.cap;
         const float hk2 = c.hk2;
-        uint32_t nf = 0, nb = 0;
+        uint32_t nf = 0, nb = 0;                 // found; stored while below max_neighbors
         if (S != kUnstaged) {
             ListWriter16 w{reinterpret_cast<uint4*>(nbr16) + i, cap};
-            const uint32_t self = s_off[uown] + (i - s_src[uown]);
+            const uint32_t self = i - s_src[uown];
             if (lds_search) {
-                // Each row range goes in chunks of 32 candidates: a branch-free
+                // Each row range goes in chunks of up to 32 candidates: a branch-free
                 // pass sets one bit per candidate within h, then the set bits
-                // are appended in order (stored while below max_neighbors).
-                uint32_t ntot = 0;
-#pragma unroll
+                // are appended in order.
+#pragma unroll 1
                 for (int r = 0; r < 9; ++r) {
                     if (row[r] == kNoRow) continue;
-                    const uint32_t e = s_off[(row[r] >> 16) + 1u];
-                    for (uint32_t l0 = s_off[row[r] & 0xffffu]; l0 < e; l0 += 32u) {
-                        const uint32_t cnt = min(e - l0, 32u);
-                        uint32_t m = 0, t = 0;
-                        for (; t + 2u <= cnt; t += 2u) {
-                            const float4 qa = s_pos[l0 + t], qb = s_pos[l0 + t + 1u];
-                            const uint32_t ia = dist2(p.x - qa.x, p.y - qa.y, p.z - qa.z) < hk2 ? 1u : 0u;
-                            const uint32_t ib = dist2(p.x - qb.x, p.y - qb.y, p.z - qb.z) < hk2 ? 2u : 0u;
-                            m |= (ia | ib) << t;
-                        }
-                        if (t < cnt) {
-                            const float4 qa = s_pos[l0 + t];
-                            m |= (dist2(p.x - qa.x, p.y - qa.y, p.z - qa.z) < hk2 ? 1u : 0u) << t;
-                        }
-                        if (self - l0 < cnt) m &= ~(1u << (self - l0));
-                        ntot += (uint32_t)__popc(m);
-                        while (m != 0u && nf < maxn) {
-                            w.push(nf, (l0 + (uint32_t)__builtin_ctz(m)) << 4);   // LDS byte offset
-                            ++nf;
-                            m &= m - 1u;
-                        }
+                    const uint32_t s0 = s_off[row[r] & 0xffffu], e = s_off[(row[r] >> 16) + 1u];
+                    for (uint32_t l0 = s0 & ~1u; l0 < e; l0 += 32u) {
+                        uint32_t m = near_mask(st, p, hk2, l0, e);
+                        if (l0 < s0) m &= ~1u;           // the position before the range
+                        if (self - l0 < 32u) m &= ~(1u << (self - l0));
+                        const uint32_t hits = (uint32_t)__popc(m);
+                        if (nf + hits > maxn) m = lowest_bits(m, nf < maxn ? maxn - nf : 0u);
+                        nf += hits;
+                        for (; m != 0u; m &= m - 1u) w.push((l0 + (uint32_t)__builtin_ctz(m)) << 4);   // LDS byte offset
                     }
                 }
-                nf = ntot;                      // stored: min(nf, max_neighbors), as below
             } else {
-#pragma unroll
+#pragma unroll 1
                 for (int r = 0; r < 9; ++r) {
                     if (row[r] == kNoRow) continue;
                     for (uint32_t u = row[r] & 0xffffu; u <= (row[r] >> 16); ++u) {
-                        const uint32_t e = s_off[u + 1u], src = s_src[u] - s_off[u];
+                        const uint32_t e = s_off[u + 1u], src = s_src[u];
+#pragma unroll 1
                         for (uint32_t l = s_off[u]; l < e; ++l) {
                             const float4 qp = pos[src + l];
                             const bool in = dist2(p.x - qp.x, p.y - qp.y, p.z - qp.z) < hk2 && l != self;
                             if (in) {
-                                if (nf < maxn) w.push(nf, l << 4);
+                                if (nf < maxn) w.push(l << 4);
                                 ++nf;
                             }
                         }
                     }
                 }
             }
-            w.finish(nf < maxn ? nf : maxn);
+            w.finish();
         } else {
             ListWriter32 w{reinterpret_cast<uint4*>(nbrf) + i, cap};
             auto scan_range = [&](uint32_t s0, uint32_t e) {
@@ -658,22 +730,22 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* 
                     const uint32_t j = INDIRECT ? perm[q] : q;
                     const float4 pj = pos[j];
                     if (dist2(p.x - pj.x, p.y - pj.y, p.z - pj.z) < hk2 && j != i) {
-                        if (nf < maxn) w.push(nf, j);
+                        if (nf < maxn) w.push(j);
                         ++nf;
                     }
                 }
             };
             if (tabled) {
-#pragma unroll
+#pragma unroll 1
                 for (int r = 0; r < 9; ++r) {
                     if (row[r] == kNoRow) continue;
                     for (uint32_t u = row[r] & 0xffffu; u <= (row[r] >> 16); ++u)
-                        scan_range(s_src[u], s_src[u] + (s_off[u + 1u] - s_off[u]));
+                        scan_range(s_src[u] + s_off[u], s_src[u] + s_off[u + 1u]);
                 }
             } else {
-                for_each_adjacent_cell(c, cx, cy, cz, [&](uint32_t nk) { scan_range(cs_f[nk], cs_f[nk + 1]); });
+                for_each_adjacent_range(c, cx, cy, cz, cs_f, scan_range);
             }
-            w.finish(nf < maxn ? nf : maxn);
+            w.finish();
         }
         const uint32_t sf = nf < maxn ? nf : maxn;
         ListWriter32 wb{reinterpret_cast<uint4*>(nbrb) + i, cap};
@@ -681,52 +753,48 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* 
             for (uint32_t j = s0; j < e; ++j) {
                 const float4 pj = bpos[j];
                 if (dist2(p.x - pj.x, p.y - pj.y, p.z - pj.z) < hk2) {
-                    if (sf + nb < maxn) wb.push(nb, j);
+                    if (sf + nb < maxn) wb.push(j);
                     ++nb;
                 }
             }
         };
         if (lds_bnd) {
-            // the row's boundary particles are one contiguous staged range;
-            // the same chunked bitmask pass as the fluid search
-            uint32_t ntot = 0;
-#pragma unroll
-            for (int r = 0; r < 9; ++r) {
-                if (row[r] == kNoRow) continue;
-                const uint32_t e = S + s_boff[(row[r] >> 16) + 1u];
-                for (uint32_t l0 = S + s_boff[row[r] & 0xffffu]; l0 < e; l0 += 32u) {
-                    const uint32_t cntc = min(e - l0, 32u);
-                    uint32_t m = 0, t = 0;
-                    for (; t + 2u <= cntc; t += 2u) {
-                        const float4 qa = s_pos[l0 + t], qb = s_pos[l0 + t + 1u];
-                        const uint32_t ia = dist2(p.x - qa.x, p.y - qa.y, p.z - qa.z) < hk2 ? 1u : 0u;
-                        const uint32_t ib = dist2(p.x - qb.x, p.y - qb.y, p.z - qb.z) < hk2 ? 2u : 0u;
-                        m |= (ia | ib) << t;
-                    }
-                    if (t < cntc) {
-                        const float4 qa = s_pos[l0 + t];
-                        m |= (dist2(p.x - qa.x, p.y - qa.y, p.z - qa.z) < hk2 ? 1u : 0u) << t;
-                    }
-                    ntot += (uint32_t)__popc(m);
-                    while (m != 0u && sf + nb < maxn) {
-                        wb.push(nb, __float_as_uint(s_pos[l0 + (uint32_t)__builtin_ctz(m)].w));
-                        ++nb;
-                        m &= m - 1u;
+            // the row's boundary particles are one contiguous staged range, in
+            // up to three runs of boundary indices (one per cell)
+            if (Sb > 0u) {
+#pragma unroll 1
+                for (int r = 0; r < 9; ++r) {
+                    if (row[r] == kNoRow) continue;
+                    const uint32_t u0 = row[r] & 0xffffu, u1 = row[r] >> 16;
+                    const uint32_t s0 = S + s_boff[u0], e = S + s_boff[u1 + 1u];
+                    if (s0 == e) continue;
+                    const uint32_t ub = min(u0 + 1u, u1), k1 = S + s_boff[ub], k2 = S + s_boff[u1];
+                    const uint32_t j0 = s_bs[u0] - S, j1 = s_bs[ub] - S, j2 = s_bs[u1] - S;
+                    for (uint32_t l0 = s0 & ~1u; l0 < e; l0 += 32u) {
+                        uint32_t m = near_mask(st, p, hk2, l0, e);
+                        if (l0 < s0) m &= ~1u;           // the position before the range
+                        const uint32_t hits = (uint32_t)__popc(m);
+                        if (sf + nb + hits > maxn) m = lowest_bits(m, sf + nb < maxn ? maxn - sf - nb : 0u);
+                        nb += hits;
+                        for (; m != 0u; m &= m - 1u) {
+                            const uint32_t k = l0 + (uint32_t)__builtin_ctz(m);
+                            wb.push(k + (k < k1 ? j0 : k < k2 ? j1 : j2));
+                        }
                     }
                 }
             }
-            nb = ntot;
         } else if (tabled) {
-#pragma unroll
+#pragma unroll 1
             for (int r = 0; r < 9; ++r) {
                 if (row[r] == kNoRow) continue;
-                for (uint32_t u = row[r] & 0xffffu; u <= (row[r] >> 16); ++u) scan_boundary(s_bs[u], s_be[u]);
+                for (uint32_t u = row[r] & 0xffffu; u <= (row[r] >> 16); ++u)
+                    scan_boundary(s_bs[u] + s_boff[u], s_bs[u] + s_boff[u + 1u]);
             }
         } else {
-            for_each_adjacent_cell(c, cx, cy, cz, [&](uint32_t nk) { scan_boundary(cs_b[nk], cs_b[nk + 1]); });
+            for_each_adjacent_range(c, cx, cy, cz, cs_b, scan_boundary);
         }
         const uint32_t sb = nb < maxn - sf ? nb : maxn - sf;
-        wb.finish(sb);
+        wb.finish();
         total = nf + nb;
         trunc = total > maxn ? 1u : 0u;
         cnt[i] = sf | (sb << 16);
@@ -736,8 +804,8 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(SimConst c, const float4* 
     }
     // the block's statistics go to part[2b], part[2b + 1] (k_nbr_finalize
     // sums them): per-wave atomics on one control line would serialise
-    const uint32_t wv[5] = {wave_max_u(total), wave_sum_u(trunc), wave_sum_u(stored_f), wave_sum_u(stored_b),
-                            wave_sum_u(stored_u32)};
+    const uint32_t wv[5] = {(uint32_t)wave_max_i((int)total), wave_total_u(trunc), wave_total_u(stored_f),
+                            wave_total_u(stored_b), wave_total_u(stored_u32)};
     const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0)
         for (int k = 0; k < 5; ++k) s_w[5 * w + k] = (int)wv[k];

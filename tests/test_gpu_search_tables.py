@@ -1,0 +1,89 @@
+"""Neighbor search: the staged search against the search without sets (every
+list form has to give the same lists in the same order) and against all pairs,
+at the edges of its tables: few particles, block remainders, spray with
+many cells a block, rows of more than 32 candidates, sets beyond the stage, a
+string of particles too long for the row masks, dense walls and truncated lists."""
+import numpy as np
+import pytest
+
+import splishsplash_for_cuda_amd as S
+from splishsplash_for_cuda_amd.scene import box_surface, fluid_block
+
+pytestmark = pytest.mark.gpu
+R = 0.025
+H = 4.0 * R
+
+
+def _jitter(x, rng, j):
+    return x + rng.uniform(-j * R, j * R, x.shape)
+
+
+def _scene(name, rng):
+    """fluid, walls, max_neighbors"""
+    box = (2.0, 2.0, 2.0)
+    walls = box_surface((0, 0, 0), box, 2 * R)
+    maxn = 128
+    if name.startswith("n="):
+        n = int(name[2:])
+        x = _jitter(fluid_block((0.05, 0.05, 0.05), (9, 9, 9), 2 * R), rng, 0.2)[:n]
+    elif name == "spray":
+        x = rng.uniform(0.05, 1.95, (3000, 3))
+    elif name == "thin spray":
+        x = rng.uniform(0.05, 1.95, (700, 3))
+    elif name == "rows over 32":
+        x = _jitter(fluid_block((0.4, 0.4, 0.4), (16, 16, 16), 1.25 * R), rng, 0.2)
+        maxn = 255
+    elif name == "sets over the stage":
+        x = _jitter(fluid_block((0.4, 0.4, 0.4), (22, 20, 21), 1.02 * R), rng, 0.2)
+        maxn = 255
+    elif name == "string":
+        walls = box_surface((0, 0, 0), (12.0, 0.4, 0.4), 2 * R)
+        x = _jitter(np.stack([np.linspace(0.1, 11.9, 900), np.full(900, 0.2), np.full(900, 0.2)], 1), rng, 0.5)
+    elif name == "dense walls":
+        walls = box_surface((0, 0, 0), (0.8, 0.8, 0.8), 0.6 * R)
+        x = _jitter(fluid_block((0.04, 0.04, 0.04), (15, 14, 13), 2 * R), rng, 0.2)
+        maxn = 255
+    else:                                       # "truncated"
+        x = _jitter(fluid_block((0.05, 0.05, 0.05), (14, 13, 12), 2 * R), rng, 0.2)
+        maxn = 21
+    return x.astype(np.float32), walls.astype(np.float32), maxn
+
+
+def _search(x, walls, maxn, mode):
+    s = S.Solver(S.default_params(particle_radius=R, max_neighbors=maxn, list_mode=mode))
+    s.upload_boundary(walls)
+    s.upload_fluid(x)
+    s.neighbor_search()
+    nf, nb, L = s.neighbors()
+    out = (s.download(S.FIELD_POS), s.download(S.FIELD_BOUNDARY_POS), nf, nb, L, s.neighbor_stats())
+    s.close()
+    return out
+
+
+@pytest.mark.parametrize("name", ["n=1", "n=2", "n=63", "n=511", "n=512", "n=513", "spray", "thin spray", "rows over 32",
+                                  "sets over the stage", "string", "dense walls", "truncated"])
+def test_search_tables(name):
+    x, walls, maxn = _scene(name, np.random.default_rng(11))
+    pos, bpos, nf, nb, L, stats = _search(x, walls, maxn, S.LISTS_AUTO)
+    _, _, gf, gb, G, gstats = _search(x, walls, maxn, S.LISTS_GLOBAL)
+    assert stats == gstats
+    assert np.array_equal(nf, gf) and np.array_equal(nb, gb) and np.array_equal(L, G)
+    # all pairs in 64 bits: equal except within rounding of the support's edge
+    p, q = pos.astype(np.float64), bpos.astype(np.float64)
+    h2 = float(np.float32(H)) ** 2
+    over = 0
+    for i in range(len(p)):
+        d, db = ((p - p[i]) ** 2).sum(1), ((q - p[i]) ** 2).sum(1)
+        d[i] = np.inf
+        edge = (np.abs(d - h2) < 1e-5 * h2).any() or (np.abs(db - h2) < 1e-5 * h2).any()
+        wf, wb = np.flatnonzero(d < h2), np.flatnonzero(db < h2)
+        over += len(wf) + len(wb) > maxn
+        if edge:
+            continue
+        got_f, got_b = L[i, :nf[i]], L[i, nf[i]:nf[i] + nb[i]]
+        if len(wf) + len(wb) <= maxn:
+            assert np.array_equal(np.sort(got_f), wf) and np.array_equal(np.sort(got_b), wb)
+        else:
+            assert len(got_f) == min(len(wf), maxn) and len(got_f) + len(got_b) == maxn
+            assert np.isin(got_f, wf).all() and np.isin(got_b, wb).all()
+    assert over > 0 or name != "truncated"
