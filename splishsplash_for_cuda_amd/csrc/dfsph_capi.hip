@@ -339,7 +339,7 @@ int ensure_tmp(Handle* h, uint32_t n)
     if (n <= h->tmp_cap && h->key) return DFSPH_OK;
     CHK(dalloc(h->key, (size_t)n + 1));     // n + 1: also class flags / ranks with a sentinel
     CHK(dalloc(h->slot, (size_t)n + 1));
-    CHK(dalloc(h->perm, n));
+    CHK(dalloc(h->perm, (size_t)n + 1));
     CHK(dalloc(h->keep, (size_t)n + 1));
     CHK(dalloc(h->rank, (size_t)n + 1));
     CHK(dalloc(h->keep8, n));
@@ -358,15 +358,25 @@ int ensure_partials(Handle* h, uint32_t n)
     return DFSPH_OK;
 }
 
-// counting sort of n points into the cell table cs (ncell+1 entries);
-// perm[k] = index of the point at sorted slot k (stable)
+// counting sort of n points into the cell table cs (ncell+1 entries): their
+// keys in key, and in perm each cell's points in an order that varies from run
+// to run (the gathers and launch_order_perm make it stable)
 int counting_sort(Handle* h, const float4* pts, uint32_t n, uint32_t* cs)
 {
     const uint32_t nc = h->c.ncell;
     dfsph::launch_cell_hist(h->s, h->c, pts, n, h->key, h->slot, h->hist);
     dfsph::launch_exclusive_scan(h->s, h->hist, cs, nc + 1, h->scan_tmp, true);   // leaves hist zeroed
     dfsph::launch_scatter_perm(h->s, h->key, h->slot, cs, n, h->perm);
-    dfsph::launch_cell_sort(h->s, cs, nc, h->perm);
+    HIPCHK(hipGetLastError());
+    return DFSPH_OK;
+}
+
+// the same with perm[k] = index of the point at sorted slot k (stable)
+int counting_order(Handle* h, const float4* pts, uint32_t n, uint32_t* cs)
+{
+    CHK(counting_sort(h, pts, n, cs));
+    dfsph::launch_order_perm(h->s, n, h->key, cs, h->perm, h->slot);   // the slots are done with
+    std::swap(h->perm, h->slot);
     HIPCHK(hipGetLastError());
     return DFSPH_OK;
 }
@@ -405,8 +415,7 @@ int place_bodies(Handle* h)
     dfsph::launch_bodies_place(h->s, h->dbody, h->x0, h->sbody, h->ns, h->braw + h->nbs, h->bvraw + h->nbs,
                                h->sforce);
     CHK(counting_sort(h, h->braw, h->nb, h->bcstart));
-    dfsph::launch_gather_f4(h->s, h->nb, h->perm, h->braw, h->bpos);
-    dfsph::launch_gather_f4(h->s, h->nb, h->perm, h->bvraw, h->bvel);
+    dfsph::launch_gather_boundary(h->s, h->nb, h->key, h->bcstart, h->perm, h->braw, h->bpos, h->bvraw, h->bvel);
     HIPCHK(hipGetLastError());
     return DFSPH_OK;
 }
@@ -423,10 +432,12 @@ int neighbor_search(Handle* h, bool sort)
         return DFSPH_OK;
     }
     const int ps = pbeg(h, DFSPH_KERNEL_SORT);
-    CHK(counting_sort(h, h->pos[h->pc], h->n, h->cstart));
-    if (sort) {
+    if (!sort) {
+        CHK(counting_order(h, h->pos[h->pc], h->n, h->cstart));
+    } else {
+        CHK(counting_sort(h, h->pos[h->pc], h->n, h->cstart));
         const int o = h->pc ^ 1, vo = h->vc ^ 1;
-        dfsph::launch_gather_fluid(h->s, h->n, h->perm, fluid_ptrs(h, h->pc, h->vc), fluid_ptrs(h, o, vo));
+        dfsph::launch_gather_fluid(h->s, h->n, h->key, h->cstart, h->perm, fluid_ptrs(h, h->pc, h->vc), fluid_ptrs(h, o, vo));
         h->pc = o;
         h->vc = vo;
     }
@@ -1109,7 +1120,7 @@ int dfsph_upload_boundary(void* hv, const float* xyz, const float* psi, uint32_t
     HIPCHK(hipMemcpyAsync(raw, P.data(), sizeof(float4) * n, hipMemcpyHostToDevice, h->s));
     int rc = counting_sort(h, raw, n, h->bcstart);
     if (rc == DFSPH_OK) {
-        dfsph::launch_gather_f4(h->s, n, h->perm, raw, h->bpos);
+        dfsph::launch_gather_boundary(h->s, n, h->key, h->bcstart, h->perm, raw, h->bpos, nullptr, nullptr);
         if (!psi) {
             float* tmp = nullptr;
             rc = dalloc(tmp, n);
@@ -1858,7 +1869,7 @@ int dfsph_open_boundary_apply(void* hv, const double* window_displacement, float
         const uint32_t n = h->n, nc = h->ob_n;
         if (nc && n) {
             // cell table of the current positions without reordering
-            CHK(counting_sort(h, h->pos[h->pc], n, h->cstart));
+            CHK(counting_order(h, h->pos[h->pc], n, h->cstart));
             uint32_t *k = h->ob_k, *r = h->ob_r, *tmp = h->ob_tmp;
             float4* vnew = h->ob_vnew;
             float4 p0;
@@ -1936,7 +1947,7 @@ int dfsph_load_fluid(void* hv, const float* xyz, uint32_t nc, float min_distance
         // moved since the last search counts where it is now)
         if (h->ns) CHK(place_bodies(h));
         const uint32_t n = h->n;
-        CHK(counting_sort(h, h->pos[h->pc], n, h->cstart));
+        CHK(counting_order(h, h->pos[h->pc], n, h->cstart));
         float4 p0;
         HIPCHK(hipMemcpyAsync(&p0, h->pos[h->pc], sizeof(float4), hipMemcpyDeviceToHost, h->s));
         CHK(sync(h));

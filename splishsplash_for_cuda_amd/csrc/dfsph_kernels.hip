@@ -256,20 +256,39 @@ __global__ void k_scatter_perm(const uint32_t* key, const uint32_t* slot, const 
 }
 
 // The arrival slots come from atomics, so the order inside a cell varies from
-// run to run (DFSPH_core_cuda.cu:1845-1846).  Sorting each cell's few entries
-// by original index makes the counting sort stable and the whole step
-// bit-reproducible.
-__global__ void k_cell_sort(const uint32_t* cstart, uint32_t ncell, uint32_t* perm)
+// run to run (DFSPH_core_cuda.cu:1845-1846).  A particle's place is its cell's
+// start plus the number of the cell's entries with a smaller original index,
+// which makes the counting sort stable and the whole step bit-reproducible.
+// The consumers of the order count it themselves, one thread per entry: the
+// cell's entries are in a cache line or two that the neighbors read too,
+// and no pass sorts them in memory (an insertion sort with a thread per cell
+// took 28 us of a 4.19 M particle search, 80 us with 200k particles where
+// spray crowds some cells).
+struct CellOrder {
+    const uint32_t* __restrict__ key;
+    const uint32_t* __restrict__ cstart;
+    const uint32_t* __restrict__ perm;   // perm: the entries of each cell in arrival order
+};
+
+__device__ __forceinline__ uint32_t ordered_place(const CellOrder& o, uint32_t i)
 {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncell) return;
-    const uint32_t s = cstart[c], e = cstart[c + 1];
-    for (uint32_t a = s + 1; a < e; ++a) {
-        const uint32_t v = perm[a];
-        uint32_t b = a;
-        while (b > s && perm[b - 1] > v) { perm[b] = perm[b - 1]; --b; }
-        perm[b] = v;
+    const uint32_t c = o.key[i], s = o.cstart[c], e = o.cstart[c + 1];
+    uint32_t rank = 0, q = s;
+    for (; q + 4u <= e; q += 4u) {
+        const uint32_t a0 = o.perm[q], a1 = o.perm[q + 1u], a2 = o.perm[q + 2u], a3 = o.perm[q + 3u];
+        rank += (a0 < i ? 1u : 0u) + (a1 < i ? 1u : 0u) + (a2 < i ? 1u : 0u) + (a3 < i ? 1u : 0u);
     }
+    for (; q < e; ++q) rank += o.perm[q] < i ? 1u : 0u;
+    return s + rank;
+}
+
+// the stable order itself, for searches and scans that read through it
+__global__ void k_order_perm(uint32_t n, CellOrder o, uint32_t* out)
+{
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const uint32_t i = o.perm[k];
+    out[ordered_place(o, i)] = i;
 }
 
 // cuda_sortData (DFSPH_core_cuda.cu:2057-2129): one gather of every persistent
@@ -286,18 +305,35 @@ __device__ __forceinline__ void copy_fluid(const FluidPtrs& a, uint32_t from, co
     b.tag[to] = a.tag[from];
 }
 
-__global__ void k_gather_fluid(uint32_t n, const uint32_t* perm, FluidPtrs in, FluidPtrs out)
+__global__ void k_gather_fluid(uint32_t n, CellOrder o, FluidPtrs in, FluidPtrs out)
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    copy_fluid(in, perm[k], out, k);
+    const uint32_t i = o.perm[k];
+    // the record is in flight while its place is counted
+    const float4 p = in.pos[i], v = in.vel[i];
+    const float ka = in.kap[i], kv = in.kapv[i], kt = in.ktot[i], kvt = in.kvtot[i];
+    const uint32_t id = in.id[i], tag = in.tag[i];
+    const uint32_t to = ordered_place(o, i);
+    out.pos[to] = p;
+    out.vel[to] = v;
+    out.kap[to] = ka;
+    out.kapv[to] = kv;
+    out.ktot[to] = kt;
+    out.kvtot[to] = kvt;
+    out.id[to] = id;
+    out.tag[to] = tag;
 }
 
-__global__ void k_gather_f4(uint32_t n, const uint32_t* perm, const float4* in, float4* out)
+// the boundary set's records (positions, and velocities when given) in cell order
+__global__ void k_gather_boundary(uint32_t n, CellOrder o, const float4* in, float4* out, const float4* vin,
+                                  float4* vout)
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    out[k] = in[perm[k]];
+    const uint32_t i = o.perm[k], to = ordered_place(o, i);
+    out[to] = in[i];
+    if (vin) vout[to] = vin[i];
 }
 
 // Appends list entries to a particle's blocked-interleaved list: entries
@@ -1794,19 +1830,22 @@ void launch_scatter_perm(hipStream_t s, const uint32_t* key, const uint32_t* slo
     if (n) k_scatter_perm<<<nblk(n), kBlock, 0, s>>>(key, slot, cstart, n, perm);
 }
 
-void launch_cell_sort(hipStream_t s, const uint32_t* cstart, uint32_t ncell, uint32_t* perm)
+void launch_order_perm(hipStream_t s, uint32_t n, const uint32_t* key, const uint32_t* cstart, const uint32_t* perm,
+                       uint32_t* out)
 {
-    k_cell_sort<<<nblk(ncell), kBlock, 0, s>>>(cstart, ncell, perm);
+    if (n) k_order_perm<<<nblk(n), kBlock, 0, s>>>(n, CellOrder{key, cstart, perm}, out);
 }
 
-void launch_gather_fluid(hipStream_t s, uint32_t n, const uint32_t* perm, const FluidPtrs& in, const FluidPtrs& out)
+void launch_gather_fluid(hipStream_t s, uint32_t n, const uint32_t* key, const uint32_t* cstart, const uint32_t* perm,
+                         const FluidPtrs& in, const FluidPtrs& out)
 {
-    if (n) k_gather_fluid<<<nblk(n), kBlock, 0, s>>>(n, perm, in, out);
+    if (n) k_gather_fluid<<<nblk(n), kBlock, 0, s>>>(n, CellOrder{key, cstart, perm}, in, out);
 }
 
-void launch_gather_f4(hipStream_t s, uint32_t n, const uint32_t* perm, const float4* in, float4* out)
+void launch_gather_boundary(hipStream_t s, uint32_t n, const uint32_t* key, const uint32_t* cstart,
+                            const uint32_t* perm, const float4* in, float4* out, const float4* vin, float4* vout)
 {
-    if (n) k_gather_f4<<<nblk(n), kBlock, 0, s>>>(n, perm, in, out);
+    if (n) k_gather_boundary<<<nblk(n), kBlock, 0, s>>>(n, CellOrder{key, cstart, perm}, in, out, vin, vout);
 }
 
 void launch_neighbors(hipStream_t s, const SimConst& c, bool indirect, const float4* pos, const uint32_t* cs_f,

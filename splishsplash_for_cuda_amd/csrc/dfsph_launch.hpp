@@ -37,9 +37,14 @@ void launch_cell_hist(hipStream_t s, const SimConst& c, const float4* pos, uint3
                       uint32_t* slot, uint32_t* hist);
 void launch_scatter_perm(hipStream_t s, const uint32_t* key, const uint32_t* slot, const uint32_t* cstart,
                          uint32_t n, uint32_t* perm);
-void launch_cell_sort(hipStream_t s, const uint32_t* cstart, uint32_t ncell, uint32_t* perm);
-void launch_gather_fluid(hipStream_t s, uint32_t n, const uint32_t* perm, const FluidPtrs& in, const FluidPtrs& out);
-void launch_gather_f4(hipStream_t s, uint32_t n, const uint32_t* perm, const float4* in, float4* out);
+// from the keys, the cell table and the scattered permutation: the stable
+// order (out must not be perm), or records moved into it
+void launch_order_perm(hipStream_t s, uint32_t n, const uint32_t* key, const uint32_t* cstart, const uint32_t* perm,
+                       uint32_t* out);
+void launch_gather_fluid(hipStream_t s, uint32_t n, const uint32_t* key, const uint32_t* cstart, const uint32_t* perm,
+                         const FluidPtrs& in, const FluidPtrs& out);
+void launch_gather_boundary(hipStream_t s, uint32_t n, const uint32_t* key, const uint32_t* cstart,
+                            const uint32_t* perm, const float4* in, float4* out, const float4* vin, float4* vout);
 void launch_neighbors(hipStream_t s, const SimConst& c, bool indirect, const float4* pos, const uint32_t* cs_f,
                       const uint32_t* perm, const float4* bpos, const uint32_t* cs_b, uint32_t n,
                       uint16_t* nbr16, uint32_t* nbrf, uint32_t* nbrb, uint32_t* cnt, uint32_t* stage_n,

@@ -87,3 +87,29 @@ def test_search_tables(name):
             assert len(got_f) == min(len(wf), maxn) and len(got_f) + len(got_b) == maxn
             assert np.isin(got_f, wf).all() and np.isin(got_b, wb).all()
     assert over > 0 or name != "truncated"
+
+
+@pytest.mark.parametrize("crowd", [0, 700])
+@pytest.mark.parametrize("n", [1, 513, 4000])
+def test_cell_order_is_stable(n, crowd):
+    """Inside a cell the sorted particles keep the order they had (here their ids),
+    also in a cell of hundreds and with ids scattered over the cells."""
+    rng = np.random.default_rng(n + crowd)
+    x = rng.uniform(0.1, 1.9, (n, 3))
+    if crowd:
+        x = np.concatenate([x, 1.0 + rng.uniform(0.0, 0.2 * H, (crowd, 3))])
+        x = x[rng.permutation(len(x))]
+    s = S.Solver(S.default_params(particle_radius=R, max_neighbors=20))
+    s.upload_boundary(box_surface((0, 0, 0), (2.0, 2.0, 2.0), 2 * R).astype(np.float32))
+    x = x.astype(np.float32)
+    s.upload_fluid(x)
+    s.neighbor_search()
+    ids, pos, inf = s.download(S.FIELD_ID), s.download(S.FIELD_POS), s.info()
+    s.close()
+    assert np.array_equal(np.sort(ids), np.arange(len(x))) and np.array_equal(pos, x[ids])
+    inv = np.float32(1.0 / inf.cell_size)
+    cell = np.floor((pos - np.array(inf.grid_origin[:], np.float32)) * inv).astype(np.int64)
+    same = (cell[1:] == cell[:-1]).all(1)
+    assert (ids[1:][same] > ids[:-1][same]).all()
+    # each cell is one run
+    assert (~same).sum() + 1 == len(np.unique(cell, axis=0))
