@@ -11,13 +11,13 @@
 // BF16 on the matrix cores (v_mfma_f32_16x16x16_bf16, FP32 accumulate);
 // biases, activations between layers and all reductions are FP32.
 //
-// Wave-level tiling: one wavefront owns 64 particles (four 16-row tiles).
 // MFMA 16x16x16 operand layout (lane l = 0..63, q = 0..3):
 //   A[i][k]: lane l holds A[l % 16][4 (l / 16) + q]
 //   B[k][n]: lane l holds B[4 (l / 16) + q][l % 16]
 //   D[i][n]: lane l holds D[4 (l / 16) + q][l % 16]
-// Activations pass between layers through LDS (bf16), which turns the D
-// layout of one layer into the A layout of the next.
+// Layers are computed transposed, H_out^T = W H_in^T, with 16 samples as the N
+// dimension: the output tile a lane holds is the B operand of the next layer's
+// matching K block.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -52,8 +52,6 @@ __device__ __forceinline__ unsigned short f2bf(float f)
     return (unsigned short)(u >> 16);
 }
 
-__device__ __forceinline__ float bf2f(unsigned short b) { return __uint_as_float(((uint32_t)b) << 16); }
-
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + __expf(-z)); }
 
 __device__ __forceinline__ float dsilu(float z)
@@ -67,28 +65,6 @@ __device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-// General strided operand access: X(r, c) = base[r * rs + c * cs] (bf16 in LDS or global)
-struct Mat {
-    const unsigned short* p;
-    int rs, cs;
-    __device__ unsigned short at(int r, int c) const { return p[r * rs + c * cs]; }
-};
-
-// One 16x16 output tile C[mt*16.., nt*16..] = sum_k A(i, k) B(k, n) over K (multiple of 16).
-__device__ __forceinline__ f32x4 gemm_tile(const Mat& A, const Mat& B, int mt, int nt, int K, f32x4 acc)
-{
-    const int l = threadIdx.x & 63;
-    const int i = mt * 16 + (l & 15), n = nt * 16 + (l & 15);
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        const int kb = k0 + 4 * (l >> 4);
-        bf16x4 a, b;
-        a[0] = (short)A.at(i, kb); a[1] = (short)A.at(i, kb + 1); a[2] = (short)A.at(i, kb + 2); a[3] = (short)A.at(i, kb + 3);
-        b[0] = (short)B.at(kb, n); b[1] = (short)B.at(kb + 1, n); b[2] = (short)B.at(kb + 2, n); b[3] = (short)B.at(kb + 3, n);
-        acc = mfma(a, b, acc);
-    }
-    return acc;
-}
-
 // Device copy of the model: padded BF16 weight matrices for the matrix cores
 // and FP32 biases / normalisation.
 struct DevModel {
@@ -96,59 +72,12 @@ struct DevModel {
     unsigned short W2[kH * kH];
     unsigned short W3[kH * kH];
     unsigned short W4[kOutPad * kH];     // [16][64], rows 2..15 zero
+    unsigned short W2t[kH * kH];         // transposed (in x out): the backward pass's A operands
+    unsigned short W3t[kH * kH];
+    unsigned short W4t[kH * kOutPad];    // [64][16], columns 2..15 zero
     float b1[kH], b2[kH], b3[kH], b4[kOutPad];
     float norm[kNNorm];
 };
-
-// Forward pass of one wavefront over 64 rows of X0 (bf16, [64][16] in LDS).
-// Writes pre-activations Z1..Z3 (FP32, may be null) and activations A1..A3
-// (bf16) to LDS, returns the two outputs of the lane's rows in y (D layout:
-// rows 4 (l/16) + q of the 16-row tiles, column l % 16 < 2 valid).
-struct WaveBufs {
-    unsigned short* X0;   // [64][16]
-    unsigned short* A1;   // [64][64]
-    unsigned short* A2;
-    unsigned short* A3;
-    float* Z1;            // [64][64] or null (inference)
-    float* Z2;
-    float* Z3;
-};
-
-__device__ void layer(const Mat& Ain, int K, const unsigned short* W, int ldw, const float* bias, float* Zout,
-                      unsigned short* Aout)
-{
-    const int l = threadIdx.x & 63;
-    const Mat B{W, 1, ldw};   // B(k, n) = W[n][k]
-    for (int mt = 0; mt < 4; ++mt)
-        for (int nt = 0; nt < 4; ++nt) {
-            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            acc = gemm_tile(Ain, B, mt, nt, K, acc);
-            const int n = nt * 16 + (l & 15);
-            for (int q = 0; q < 4; ++q) {
-                const int r = mt * 16 + 4 * (l >> 4) + q;
-                const float z = acc[q] + bias[n];
-                if (Zout) Zout[r * kH + n] = z;
-                Aout[r * kH + n] = f2bf(silu(z));
-            }
-        }
-}
-
-__device__ void forward_wave(const DevModel& M, const WaveBufs& w, float out[4][4])
-{
-    const int l = threadIdx.x & 63;
-    layer(Mat{w.X0, kInPad, 1}, kInPad, M.W1, kInPad, M.b1, w.Z1, w.A1);
-    __syncthreads();
-    layer(Mat{w.A1, kH, 1}, kH, M.W2, kH, M.b2, w.Z2, w.A2);
-    __syncthreads();
-    layer(Mat{w.A2, kH, 1}, kH, M.W3, kH, M.b3, w.Z3, w.A3);
-    __syncthreads();
-    const Mat B{M.W4, 1, kH};
-    for (int mt = 0; mt < 4; ++mt) {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        acc = gemm_tile(Mat{w.A3, kH, 1}, B, mt, 0, kH, acc);
-        for (int q = 0; q < 4; ++q) out[mt][q] = acc[q] + M.b4[l & 15];
-    }
-}
 
 // ---------------------------------------------------------------- inference
 // x: [n][12] raw features (FP32); output o of row r goes to y[r * ystride + o * ocol]
@@ -278,167 +207,234 @@ static uint32_t infer_grid(uint32_t n)
 }
 
 // ---------------------------------------------------------------- training
-// One wavefront per 64 samples: forward, loss 0.5 |y - t|^2 / n_total, backward
-// through the four layers; the per-wave parameter gradient (flat FP32 layout)
-// goes to partial[blockIdx.x][kNParam] and the wave's loss to loss[blockIdx.x].
-__global__ __launch_bounds__(64) void k_mlp_grad(const DevModel* __restrict__ Mg, const float* __restrict__ x,
-                                                  const float* __restrict__ t, const uint32_t* __restrict__ idx,
-                                                  uint32_t n, float inv_total, int normalise,
-                                                  float* __restrict__ partial, float* __restrict__ loss)
+
+// row `row` of a mini-batch: a counter-based hash (splitmix64) of the training set
+__device__ __forceinline__ uint32_t batch_sample(uint64_t seed, uint32_t row, uint32_t nsrc)
 {
-    __shared__ unsigned short X0[64 * kInPad];
-    __shared__ unsigned short A1[64 * kH], A2[64 * kH], A3[64 * kH];
-    __shared__ float Z1[64 * kH], Z2[64 * kH], Z3[64 * kH];
-    __shared__ unsigned short D[64 * kH];      // dZ (bf16) of the current layer
-    __shared__ unsigned short DY[64 * kOutPad];
-    __shared__ float lsum[64];
+    uint64_t z = seed + 0x9e3779b97f4a7c15ull * (uint64_t)(row + 1);
+    z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+    z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+    z ^= z >> 31;
+    return (uint32_t)(z % nsrc);
+}
+
+// Forward, loss 0.5 |y - t|^2 inv_total, and backward of n samples (rows of x and
+// t, or, with nsrc > 0, rows drawn from nsrc by batch_sample), 64 a block.  Its
+// parameter gradient (flat FP32 layout) goes to partial[blockIdx.x][kNParam] and
+// its loss to loss[blockIdx.x].
+//
+// A mini-batch of 4096 is 64 blocks, so a block's time is its chain of layers:
+// 16 wavefronts share it, four per tile of 16 samples, each computing 16 of a
+// layer's 64 features.  Activations and their gradients pass between a
+// tile's wavefronts through LDS in the operand layout (ex), and once more with
+// a feature's 16 samples together (tr_*), the operands of the weight
+// gradients (K = samples), whose 16 x 16 tiles the wavefronts then share.
+// The sums have the order of one wavefront taking the 64 samples in turn (as a
+// mini-batch took 47 us; now 18): samples in K, then blocks, then wavefronts.
+constexpr int kGradBlock = 1024, kGradSamples = 64;
+
+__global__ __launch_bounds__(kGradBlock) void k_mlp_grad(const DevModel* __restrict__ Mg, const float* __restrict__ x,
+                                                         const float* __restrict__ t, uint32_t n, uint32_t nsrc,
+                                                         uint64_t seed, float inv_total, int normalise,
+                                                         float* __restrict__ partial, float* __restrict__ loss)
+{
+    __shared__ bf16x4 ex[5][4][4][64];                  // h1, h2, h3, dz3, dz2 of each tile
+    __shared__ __align__(8) unsigned short tr_h[3][4][kH][16], tr_d[3][4][kH][16], tr_x[4][kInPad][16],
+        tr_y[4][kOutPad][16];
+    __shared__ float s_e2[kOut][kGradSamples];          // e^2 / 2 of each output
     const DevModel& M = *Mg;
-    const int l = threadIdx.x;
-    const uint32_t base = blockIdx.x * 64u;
-    const uint32_t row = base + l;
+    const int l = threadIdx.x & 63, W = threadIdx.x >> 6, T = W >> 2, w = W & 3;
+    const int r = l & 15, g = l >> 4;                   // sample column, 4-row group
+    const int row0 = w * 16 + 4 * g;                    // the lane's first feature
+    const uint32_t row = blockIdx.x * kGradSamples + T * 16u + (uint32_t)r;
     const bool valid = row < n;
-    const uint32_t src = valid ? (idx ? idx[row] : row) : 0u;
-    for (int k = 0; k < kInPad; ++k) {
-        float v = 0.0f;
-        if (k < kIn && valid) {
-            v = x[(size_t)src * kIn + k];
-            if (normalise) v = (v - M.norm[k]) / M.norm[kIn + k];
-        }
-        X0[l * kInPad + k] = f2bf(v);
+    const uint32_t src = !valid ? 0u : nsrc ? batch_sample(seed, row, nsrc) : row;
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (valid && g < 3) v = *reinterpret_cast<const float4*>(x + (size_t)src * kIn + 4 * g);
+    float tv[kOut] = {0.0f, 0.0f};
+    if (valid && g == 0) {
+#pragma unroll
+        for (int o = 0; o < kOut; ++o) tv[o] = t[(size_t)src * kOut + o];
     }
-    __syncthreads();
-    WaveBufs w{X0, A1, A2, A3, Z1, Z2, Z3};
-    float out[4][4];
-    forward_wave(M, w, out);
-    // dY = (y - t) / n_total for the valid rows (columns 0, 1), zero elsewhere
-    const int o = l & 15;
-    float lacc = 0.0f;
-    for (int mt = 0; mt < 4; ++mt)
-        for (int q = 0; q < 4; ++q) {
-            const int r = mt * 16 + 4 * (l >> 4) + q;
-            float d = 0.0f;
-            if (o < kOut && base + r < n) {
-                const uint32_t s = idx ? idx[base + r] : base + r;
-                float tv = t[(size_t)s * kOut + o];
-                if (normalise) tv = (tv - M.norm[2 * kIn + o]) / M.norm[2 * kIn + kOut + o];
-                const float e = out[mt][q] - tv;
-                lacc += 0.5f * e * e * inv_total;
-                d = e * inv_total;
-            }
-            DY[r * kOutPad + o] = f2bf(d);
-        }
-    lsum[l] = lacc;
-    __syncthreads();
-    if (l == 0) {
-        float s = 0.0f;
-        for (int k = 0; k < 64; ++k) s += lsum[k];
-        loss[blockIdx.x] = s;
+    const bf16x4 w1 = frag8(M.W1 + (w * 16 + r) * kInPad + 4 * g), w4t = frag8(M.W4t + (w * 16 + r) * kOutPad + 4 * g);
+    bf16x4 w2[4], w3[4], w4[4], w3t[4], w2t[4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+        w2[kt] = frag8(M.W2 + (w * 16 + r) * kH + kt * 16 + 4 * g);
+        w3[kt] = frag8(M.W3 + (w * 16 + r) * kH + kt * 16 + 4 * g);
+        w4[kt] = frag8(M.W4 + r * kH + kt * 16 + 4 * g);
+        w3t[kt] = frag8(M.W3t + (w * 16 + r) * kH + kt * 16 + 4 * g);
+        w2t[kt] = frag8(M.W2t + (w * 16 + r) * kH + kt * 16 + 4 * g);
     }
-    float* g = partial + (size_t)blockIdx.x * kNParam;
-    // bias gradients are column sums of dZ: done in FP32 from the bf16 dZ rows
-    auto col_sum_store = [&](const unsigned short* Dm, int ld, int ncol, float* dst) {
-        for (int c = l; c < ncol; c += 64) {
-            float s = 0.0f;
-            for (int r = 0; r < 64; ++r) s += bf2f(Dm[r * ld + c]);
-            dst[c] = s;
-        }
+    const f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+    auto put = [&](unsigned short (*tr)[16], int at, const bf16x4& b) {    // the lane's four rows of column r
+#pragma unroll
+        for (int q = 0; q < 4; ++q) tr[at + q][r] = (unsigned short)b[q];
     };
-    // weight gradient dW[o][k] = sum_s dZ[s][o] Aprev[s][k]: M = out, N = in, K = samples
-    auto weight_grad = [&](const unsigned short* Dm, int ldd, int nout_tiles, int nout, const unsigned short* Ap,
-                           int lda, int nin_tiles, int nin, float* dst) {
-        const Mat At{Dm, 1, ldd};     // A(i = out, k = sample) = dZ[sample][out]
-        const Mat Bs{Ap, lda, 1};     // B(k = sample, n = in) = Aprev[sample][in]
-        for (int mt = 0; mt < nout_tiles; ++mt)
-            for (int nt = 0; nt < nin_tiles; ++nt) {
-                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc = gemm_tile(At, Bs, mt, nt, 64, acc);
-                const int ci = nt * 16 + (l & 15);
-                for (int q = 0; q < 4; ++q) {
-                    const int ro = mt * 16 + 4 * (l >> 4) + q;
-                    if (ro < nout && ci < nin) dst[ro * nin + ci] = acc[q];
-                }
-            }
+    auto samples = [&](const unsigned short (*tr)[16], int at) { return frag8(&tr[at][4 * g]); };
+    auto product = [&](const bf16x4* wt, int k) {                          // rows of W H, H in ex[k]
+        f32x4 a = zero;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) a = mfma(wt[kt], ex[k][T][kt][l], a);
+        return a;
     };
-    // input gradient dA[s][k] = sum_o dZ[s][o] W[o][k]: M = samples, N = in, K = out
-    auto input_grad_to_dz = [&](const unsigned short* Dm, int ldd, int kout, const unsigned short* W, int ldw,
-                                const float* Zprev, unsigned short* Dout) {
-        const Mat A{Dm, ldd, 1};      // A(i = sample, k = out)
-        const Mat B{W, ldw, 1};       // B(k = out, n = in) = W[out][in]
-        for (int mt = 0; mt < 4; ++mt)
-            for (int nt = 0; nt < 4; ++nt) {
-                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc = gemm_tile(A, B, mt, nt, kout, acc);
-                const int c = nt * 16 + (l & 15);
-                for (int q = 0; q < 4; ++q) {
-                    const int r = mt * 16 + 4 * (l >> 4) + q;
-                    Dout[r * kH + c] = f2bf(acc[q] * dsilu(Zprev[r * kH + c]));
-                }
-            }
+    auto act = [&](f32x4& z, const float* b, int k) {                      // z += b, h = silu(z)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) z[q] += b[row0 + q];
+        const bf16x4 h = pack_bf16(silu(z[0]), silu(z[1]), silu(z[2]), silu(z[3]));
+        ex[k][T][w][l] = h;
+        put(tr_h[k][T], row0, h);
     };
-    // layer 4
-    weight_grad(DY, kOutPad, 1, kOut, A3, kH, 4, kH, g + oW4);
-    if (l < kOut) {
-        float s = 0.0f;
-        for (int r = 0; r < 64; ++r) s += bf2f(DY[r * kOutPad + l]);
-        g[ob4 + l] = s;
+    auto back = [&](const f32x4& d, const f32x4& z) {
+        return pack_bf16(d[0] * dsilu(z[0]), d[1] * dsilu(z[1]), d[2] * dsilu(z[2]), d[3] * dsilu(z[3]));
+    };
+    if (valid && normalise && g < 3) {
+        const float* mu = M.norm + 4 * g;
+        const float* sg = M.norm + kIn + 4 * g;
+        v = make_float4((v.x - mu[0]) / sg[0], (v.y - mu[1]) / sg[1], (v.z - mu[2]) / sg[2], (v.w - mu[3]) / sg[3]);
     }
-    input_grad_to_dz(DY, kOutPad, kOutPad, M.W4, kH, Z3, D);
+    const bf16x4 xb = pack_bf16(v.x, v.y, v.z, v.w);
+    if (w == 0) put(tr_x[T], 4 * g, xb);
+    f32x4 z1 = mfma(w1, xb, zero);
+    act(z1, M.b1, 0);
     __syncthreads();
-    // layer 3
-    weight_grad(D, kH, 4, kH, A2, kH, 4, kH, g + oW3);
-    col_sum_store(D, kH, kH, g + ob3);
+    f32x4 z2 = product(w2, 0);
+    act(z2, M.b2, 1);
     __syncthreads();
-    {
-        // dZ2 needs D (= dZ3) as input while D is overwritten: stage through A3
-        for (int e = l; e < 64 * kH; e += 64) A3[e] = D[e];
-        __syncthreads();
-        input_grad_to_dz(A3, kH, kH, M.W3, kH, Z2, D);
-        __syncthreads();
+    f32x4 z3 = product(w3, 1);
+    act(z3, M.b3, 2);
+    __syncthreads();
+    // every wavefront forms its tile's outputs (rows 0 and 1) and dY = (y - t) inv_total
+    const f32x4 y = product(w4, 2);
+    float d[kOut] = {0.0f, 0.0f}, e2[kOut] = {0.0f, 0.0f};
+    if (valid && g == 0) {
+#pragma unroll
+        for (int o = 0; o < kOut; ++o) {
+            if (normalise) tv[o] = (tv[o] - M.norm[2 * kIn + o]) / M.norm[2 * kIn + kOut + o];
+            const float e = (y[o] + M.b4[o]) - tv[o];
+            e2[o] = 0.5f * e * e;
+            d[o] = e * inv_total;
+        }
     }
-    // layer 2
-    weight_grad(D, kH, 4, kH, A1, kH, 4, kH, g + oW2);
-    col_sum_store(D, kH, kH, g + ob2);
-    __syncthreads();
-    {
-        for (int e = l; e < 64 * kH; e += 64) A3[e] = D[e];
-        __syncthreads();
-        input_grad_to_dz(A3, kH, kH, M.W2, kH, Z1, D);
-        __syncthreads();
+    const bf16x4 dy = pack_bf16(d[0], d[1], 0.0f, 0.0f);
+    if (w == 0) {
+        put(tr_y[T], 4 * g, dy);
+        if (g == 0) { s_e2[0][T * 16 + r] = e2[0]; s_e2[1][T * 16 + r] = e2[1]; }
     }
-    // layer 1 (inputs: 12 used columns of X0)
-    weight_grad(D, kH, 4, kH, X0, kInPad, 1, kIn, g + oW1);
-    col_sum_store(D, kH, kH, g + ob1);
+    const bf16x4 d3 = back(mfma(w4t, dy, zero), z3);
+    ex[3][T][w][l] = d3;
+    put(tr_d[2][T], row0, d3);
+    __syncthreads();
+    const bf16x4 d2 = back(product(w3t, 3), z2);
+    ex[4][T][w][l] = d2;
+    put(tr_d[1][T], row0, d2);
+    __syncthreads();
+    put(tr_d[0][T], row0, back(product(w2t, 4), z1));
+    __syncthreads();
+    // dW[o][k] = sum_s dZ[s][o] H[s][k], a 16 x 16 tile of W2 and of W3 a
+    // wavefront; W1, W4 and the biases go to four each
+    const int mt = W >> 2, nt = W & 3;
+    float* out = partial + (size_t)blockIdx.x * kNParam;
+    f32x4 g2 = zero, g3 = zero, gx = zero;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        g2 = mfma(samples(tr_d[1][k], mt * 16 + r), samples(tr_h[0][k], nt * 16 + r), g2);
+        g3 = mfma(samples(tr_d[2][k], mt * 16 + r), samples(tr_h[1][k], nt * 16 + r), g3);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        out[oW2 + (mt * 16 + 4 * g + q) * kH + nt * 16 + r] = g2[q];
+        out[oW3 + (mt * 16 + 4 * g + q) * kH + nt * 16 + r] = g3[q];
+    }
+    if (mt == 0) {                                      // W1, rows of tile nt
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gx = mfma(samples(tr_d[0][k], nt * 16 + r), samples(tr_x[k], r), gx);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (r < kIn) out[oW1 + (nt * 16 + 4 * g + q) * kIn + r] = gx[q];
+    } else if (mt == 1) {                               // W4, columns of tile nt
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gx = mfma(samples(tr_y[k], r), samples(tr_h[2][k], nt * 16 + r), gx);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (4 * g + q < kOut) out[oW4 + (4 * g + q) * kH + nt * 16 + r] = gx[q];
+    } else if (mt == 2) {                               // biases: a lane a feature, the samples in turn
+        const int rows = nt < 3 ? kH : kOut;
+        if (l < rows) {
+            float sum = 0.0f;
+            for (int k = 0; k < 4; ++k) {
+                const unsigned short* p = nt < 3 ? tr_d[nt][k][l] : tr_y[k][l];
+#pragma unroll
+                for (int q = 0; q < 16; ++q) sum += __uint_as_float((uint32_t)p[q] << 16);
+            }
+            out[(nt == 0 ? ob1 : nt == 1 ? ob2 : nt == 2 ? ob3 : ob4) + l] = sum;
+        }
+    } else if (nt == 0 && l < 8) {                      // loss: output l & 1 of the samples 4 (l / 2) .. + 3 of each tile
+        float sum = 0.0f;
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sum = __builtin_fmaf(s_e2[l & 1][k * 16 + 4 * (l >> 1) + q], inv_total, sum);
+        float all = __shfl(sum, 0, 64);
+        for (int k = 1; k < 8; ++k) all += __shfl(sum, k, 64);
+        if (l == 0) loss[blockIdx.x] = all;
+    }
 }
 
-// fixed-order sum of the per-wave partial gradients and losses
-__global__ void k_mlp_reduce(const float* __restrict__ partial, const float* __restrict__ loss, uint32_t nparts,
-                             float* __restrict__ grad, float* __restrict__ loss_out)
+static uint32_t grad_grid(uint32_t n) { return (n + kGradSamples - 1) / kGradSamples; }
+
+// One parameter of the flat layout into the model's copies.
+__device__ __forceinline__ void pack_param(DevModel* M, uint32_t p, float w)
 {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < (uint32_t)kNParam) {
-        float s = 0.0f;
-        for (uint32_t b = 0; b < nparts; ++b) s += partial[(size_t)b * kNParam + p];
-        grad[p] = s;
-    }
-    if (p == 0) {
-        float s = 0.0f;
-        for (uint32_t b = 0; b < nparts; ++b) s += loss[b];
-        *loss_out = s;
-    }
+    const int q = (int)p;
+    if (q < ob1) { M->W1[(q / kIn) * kInPad + q % kIn] = f2bf(w); }
+    else if (q < oW2) { M->b1[q - ob1] = w; }
+    else if (q < ob2) { const int e = q - oW2; M->W2[e] = f2bf(w); M->W2t[(e % kH) * kH + e / kH] = f2bf(w); }
+    else if (q < oW3) { M->b2[q - ob2] = w; }
+    else if (q < ob3) { const int e = q - oW3; M->W3[e] = f2bf(w); M->W3t[(e % kH) * kH + e / kH] = f2bf(w); }
+    else if (q < oW4) { M->b3[q - ob3] = w; }
+    else if (q < ob4) { const int e = q - oW4; M->W4[e] = f2bf(w); M->W4t[(e % kH) * kOutPad + e / kH] = f2bf(w); }
+    else { M->b4[q - ob4] = w; }
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master weights, then refresh the BF16 copies
-__global__ void k_mlp_adam(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-                           const float* __restrict__ g, float lr, float b1, float b2, float eps, float c1, float c2)
+// The blocks' partial gradients and losses summed in turn (many loads in flight),
+// a thread a parameter, then either the gradient stored (grad) or one Adam
+// step (Kingma & Ba 2015) on the FP32 master weights and their copies in the
+// model.  The block after the last parameters sums the losses.
+struct AdamArgs {
+    float *w, *m, *v;
+    float lr, b1, b2, eps, c1, c2;
+};
+constexpr uint32_t kUpdateBlock = 64, kUpdateGrid = (kNParam + kUpdateBlock - 1) / kUpdateBlock + 1;
+
+__global__ __launch_bounds__(kUpdateBlock) void k_mlp_update(const float* __restrict__ partial,
+                                                             const float* __restrict__ loss, uint32_t nparts,
+                                                             float* __restrict__ grad, AdamArgs a,
+                                                             DevModel* __restrict__ M, float* __restrict__ loss_out)
 {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (uint32_t)kNParam) return;
-    const float gi = g[p];
-    const float mi = b1 * m[p] + (1.0f - b1) * gi;
-    const float vi = b2 * v[p] + (1.0f - b2) * gi * gi;
-    m[p] = mi;
-    v[p] = vi;
-    w[p] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+    const bool losses = blockIdx.x == kUpdateGrid - 1u;
+    const uint32_t p = losses ? 0u : blockIdx.x * kUpdateBlock + threadIdx.x;
+    if (p >= (uint32_t)kNParam || (losses && threadIdx.x != 0u)) return;
+    const float* part = losses ? loss : partial + p;
+    const size_t stride = losses ? 1u : (size_t)kNParam;
+    float s = 0.0f;
+    uint32_t b = 0;
+    for (; b + 32u <= nparts; b += 32u) {
+        float u[32];
+#pragma unroll
+        for (uint32_t k = 0; k < 32u; ++k) u[k] = part[(size_t)(b + k) * stride];
+#pragma unroll
+        for (uint32_t k = 0; k < 32u; ++k) s += u[k];
+    }
+    for (; b < nparts; ++b) s += part[(size_t)b * stride];
+    if (losses) { *loss_out = s; return; }
+    if (grad) { grad[p] = s; return; }
+    const float mi = a.b1 * a.m[p] + (1.0f - a.b1) * s;
+    const float vi = a.b2 * a.v[p] + (1.0f - a.b2) * s * s;
+    a.m[p] = mi;
+    a.v[p] = vi;
+    const float wn = a.w[p] - a.lr * (mi * a.c1) / (sqrtf(vi * a.c2) + a.eps);
+    a.w[p] = wn;
+    pack_param(M, p, wn);
 }
 
 __global__ void k_mlp_pack(const float* __restrict__ w, const float* __restrict__ norm, DevModel* __restrict__ M)
@@ -449,12 +445,13 @@ __global__ void k_mlp_pack(const float* __restrict__ w, const float* __restrict_
         M->W1[t] = k < kIn ? f2bf(w[oW1 + o * kIn + k]) : 0;
     }
     if (t < (uint32_t)(kH * kH)) {
-        M->W2[t] = f2bf(w[oW2 + t]);
-        M->W3[t] = f2bf(w[oW3 + t]);
+        const uint32_t tt = (t % kH) * kH + t / kH;
+        M->W2[t] = M->W2t[tt] = f2bf(w[oW2 + t]);
+        M->W3[t] = M->W3t[tt] = f2bf(w[oW3 + t]);
     }
     if (t < (uint32_t)(kOutPad * kH)) {
         const int o = t / kH;
-        M->W4[t] = o < kOut ? f2bf(w[oW4 + t]) : 0;
+        M->W4[t] = M->W4t[(t % kH) * kOutPad + o] = o < kOut ? f2bf(w[oW4 + t]) : 0;
     }
     if (t < (uint32_t)kH) {
         M->b1[t] = w[ob1 + t];
@@ -486,11 +483,9 @@ struct MlpState {
     float* ds_x = nullptr;
     float* ds_t = nullptr;
     uint32_t ds_cap = 0, ds_n = 0, ds_stride = 1;
-    uint32_t* idx = nullptr;
-    uint32_t idx_cap = 0;
     ~MlpState()
     {
-        void* ps[] = {model, w, m, v, grad, norm, partial, lossp, loss, feat, pred, kvws, ds_x, ds_t, idx};
+        void* ps[] = {model, w, m, v, grad, norm, partial, lossp, loss, feat, pred, kvws, ds_x, ds_t};
         for (void* p : ps)
             if (p) (void)hipFree(p);
     }
@@ -672,7 +667,7 @@ int dfsph_mlp_loss_grad(void* handle, const float* x, const float* t, uint32_t n
     if (!m->loaded) return mfail(DFSPH_ERR_NO_MODEL, "no model parameters set");
     if (n == 0) return mfail(DFSPH_ERR_ARG, "no samples");
     hipStream_t s = dfsph::handle_view(handle).s;
-    const uint32_t nb = (n + 63) / 64;
+    const uint32_t nb = dfsph::grad_grid(n);
     float *dx = nullptr, *dt = nullptr, *part = nullptr, *lp = nullptr;
     int rc = malloc_dev(dx, (size_t)n * dfsph::kIn);
     if (!rc) rc = malloc_dev(dt, (size_t)n * dfsph::kOut);
@@ -681,8 +676,10 @@ int dfsph_mlp_loss_grad(void* handle, const float* x, const float* t, uint32_t n
     if (!rc) {
         (void)hipMemcpyAsync(dx, x, sizeof(float) * n * dfsph::kIn, hipMemcpyHostToDevice, s);
         (void)hipMemcpyAsync(dt, t, sizeof(float) * n * dfsph::kOut, hipMemcpyHostToDevice, s);
-        dfsph::k_mlp_grad<<<nb, 64, 0, s>>>(m->model, dx, dt, nullptr, n, 1.0f / (float)n, normalise, part, lp);
-        dfsph::k_mlp_reduce<<<(dfsph::kNParam + 255) / 256, 256, 0, s>>>(part, lp, nb, m->grad, m->loss);
+        dfsph::k_mlp_grad<<<nb, dfsph::kGradBlock, 0, s>>>(m->model, dx, dt, n, 0u, 0ull, 1.0f / (float)n, normalise, part,
+                                                           lp);
+        dfsph::k_mlp_update<<<dfsph::kUpdateGrid, dfsph::kUpdateBlock, 0, s>>>(part, lp, nb, m->grad,
+                                                                                    dfsph::AdamArgs{}, nullptr, m->loss);
         float l = 0.0f;
         (void)hipMemcpyAsync(grad, m->grad, sizeof(float) * dfsph::kNParam, hipMemcpyDeviceToHost, s);
         (void)hipMemcpyAsync(&l, m->loss, sizeof(float), hipMemcpyDeviceToHost, s);
@@ -743,18 +740,6 @@ int mlp_harvest_step(MlpState* m, hipStream_t s, const DevTime* t, uint32_t n, c
     const uint32_t add = (n + stride - 1) / stride;
     m->ds_n = m->ds_n + add > m->ds_cap ? m->ds_cap : m->ds_n + add;
     return DFSPH_OK;
-}
-
-// sample indices of one training batch: a counter-based hash (splitmix64)
-__global__ void k_batch_indices(uint32_t* idx, uint32_t batch, uint32_t n, uint64_t seed)
-{
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= batch) return;
-    uint64_t z = seed + 0x9e3779b97f4a7c15ull * (uint64_t)(b + 1);
-    z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
-    z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-    z ^= z >> 31;
-    idx[b] = (uint32_t)(z % n);
 }
 
 }  // namespace dfsph
@@ -859,30 +844,24 @@ int dfsph_mlp_train(void* handle, uint32_t steps, uint32_t batch, float lr, uint
     if (m->ds_n == 0) return mfail(DFSPH_ERR_STATE, "training set is empty");
     if (batch == 0 || batch % 64) return mfail(DFSPH_ERR_ARG, "batch must be a positive multiple of 64");
     hipStream_t s = dfsph::handle_view(handle).s;
-    const uint32_t nb = batch / 64;
+    const uint32_t nb = dfsph::grad_grid(batch);
     if (nb > m->partial_cap) {
         if (int rc = malloc_dev(m->partial, (size_t)nb * dfsph::kNParam)) return rc;
         if (int rc = malloc_dev(m->lossp, nb)) return rc;
         m->partial_cap = nb;
     }
-    if (batch > m->idx_cap) {
-        if (int rc = malloc_dev(m->idx, batch)) return rc;
-        m->idx_cap = batch;
-    }
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     for (uint32_t it = 0; it < steps; ++it) {
-        dfsph::k_batch_indices<<<(batch + 255) / 256, 256, 0, s>>>(m->idx, batch, m->ds_n,
-                                                                   ((uint64_t)seed << 32) ^ (uint64_t)it * 0x632be59bd9b4e019ull);
-        dfsph::k_mlp_grad<<<nb, 64, 0, s>>>(m->model, m->ds_x, m->ds_t, m->idx, batch, 1.0f / (float)batch, 1,
-                                            m->partial, m->lossp);
-        dfsph::k_mlp_reduce<<<(dfsph::kNParam + 255) / 256, 256, 0, s>>>(m->partial, m->lossp, nb, m->grad, m->loss);
+        dfsph::k_mlp_grad<<<nb, dfsph::kGradBlock, 0, s>>>(m->model, m->ds_x, m->ds_t, batch, m->ds_n,
+                                                           ((uint64_t)seed << 32) ^ (uint64_t)it * 0x632be59bd9b4e019ull,
+                                                           1.0f / (float)batch, 1, m->partial, m->lossp);
         m->adam_t++;
         const float c1 = 1.0f / (1.0f - std::pow(b1, (float)m->adam_t));
         const float c2 = 1.0f / (1.0f - std::pow(b2, (float)m->adam_t));
         const float lr_t = lr * (1.0f - 0.9f * (float)it / (float)(steps > 1 ? steps - 1 : 1));
-        dfsph::k_mlp_adam<<<(dfsph::kNParam + 255) / 256, 256, 0, s>>>(m->w, m->m, m->v, m->grad, lr_t, b1, b2, eps,
-                                                                       c1, c2);
-        if (int rc = pack(m, s)) return rc;
+        dfsph::k_mlp_update<<<dfsph::kUpdateGrid, dfsph::kUpdateBlock, 0, s>>>(
+            m->partial, m->lossp, nb, nullptr, dfsph::AdamArgs{m->w, m->m, m->v, lr_t, b1, b2, eps, c1, c2}, m->model,
+            m->loss);
         if (it == 0 && loss_first) MHIP(hipMemcpyAsync(loss_first, m->loss, sizeof(float), hipMemcpyDeviceToHost, s));
         if (it + 1 == steps && loss_last) MHIP(hipMemcpyAsync(loss_last, m->loss, sizeof(float), hipMemcpyDeviceToHost, s));
     }

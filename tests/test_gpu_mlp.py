@@ -88,3 +88,49 @@ def test_normalization_is_scale_free():
     assert sd[5] == pytest.approx(1.0)
     np.testing.assert_allclose(tmu, t.astype(np.float64).mean(0), rtol=1e-4)
     np.testing.assert_allclose(tsd, t.astype(np.float64).std(0), rtol=1e-3)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 129])
+def test_mlp_gradient_of_ragged_sample_counts(oracle_mod, n):
+    """Sample counts at the edges of the gradient kernel's tiles of 16 and blocks of 64
+    (the tolerances of this file)."""
+    p = _params(8)
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(n, 12)).astype(np.float32)
+    t = rng.normal(size=(n, 2)).astype(np.float32)
+    s = S.Solver()
+    s.mlp_set_params(p.astype(np.float32))
+    loss, g = s.mlp_loss_grad(x, t)
+    loss_o, g_o = oracle_mod.mlp_loss_grad(p, x, t)
+    assert loss == pytest.approx(loss_o, rel=2e-2)
+    off = np.cumsum([0] + [int(np.prod(z)) for z in SIZES])
+    for k in range(len(SIZES)):
+        a, b = g[off[k]:off[k + 1]], g_o[off[k]:off[k + 1]]
+        assert np.linalg.norm(a - b) < 5e-2 * np.linalg.norm(b), (k, n)
+
+
+@pytest.mark.parametrize("n, batch", [(1, 64), (1000, 64), (777, 192), (5000, 4096)])
+def test_training_batches_are_the_hashed_rows(n, batch):
+    """The first batch's loss is the loss of the rows splitmix64 draws, by the same
+    kernel: equal to the last bit."""
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(n, 12)).astype(np.float32)
+    t = rng.normal(size=(n, 2)).astype(np.float32)
+    s = S.Solver()
+    s.mlp_set_params(_params(9).astype(np.float32))
+    s.mlp_dataset_upload(x, t)
+    if n > 1:
+        s.mlp_fit_normalization()
+    seed = 12345
+    z = (np.uint64(seed << 32) + np.uint64(0x9e3779b97f4a7c15) * np.arange(1, batch + 1, dtype=np.uint64))
+    z = (z ^ (z >> np.uint64(30))) * np.uint64(0xbf58476d1ce4e5b9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94d049bb133111eb)
+    rows = ((z ^ (z >> np.uint64(31))) % np.uint64(n)).astype(np.int64)
+    loss, g = s.mlp_loss_grad(x[rows], t[rows], normalise=True)
+    p0, _ = s.mlp_get_params()
+    first, last = s.mlp_train(1, batch, 1e-3, seed)
+    assert np.float32(loss) == np.float32(first) == np.float32(last)
+    # Adam's first step moves each parameter against its gradient by lr (eps aside)
+    p1, _ = s.mlp_get_params()
+    big = np.abs(g) > 1e-4
+    np.testing.assert_allclose((p0 - p1)[big], 1e-3 * np.sign(g[big]), rtol=2e-3)
