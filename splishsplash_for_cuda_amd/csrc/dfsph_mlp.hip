@@ -201,13 +201,16 @@ __global__ __launch_bounds__(kInferBlock, 3) void k_mlp_infer(const DevModel* __
 
 // Each wavefront loads all weights (20 KB) before its first tile, so small calls
 // get two wavefronts per SIMD (150k particles: 41 us with 2048 blocks, 24 with
-// 768, 22 with 512) and more join from 20 tiles each, where the load is paid off
-// and they even out the end (4.2 M: 322 us with 512, 295 with 768, 289 with 2048).
+// 768, 22 with 512).  From 20 tiles a wavefront the third resident one joins
+// (1 M: 88 us with 512, 83 with 768; 781 blocks start a second round: 106), and
+// very large calls take more rounds, which even out the end (4.2 M: 322 us with
+// 512, 295 with 768, 289 with 2048).
 static uint32_t infer_grid(uint32_t n)
 {
     const uint32_t tiles = (n + 15) / 16, per_block = kInferBlock / 64;
     const uint32_t need = (tiles + per_block - 1) / per_block;
-    return std::max(1u, std::min(need, std::clamp(need / 20u, 512u, 2048u)));
+    if (need >= 20u * 2048u) return 2048u;
+    return std::max(1u, std::min(need, std::clamp(need / 20u, 512u, 768u)));
 }
 
 // ---------------------------------------------------------------- training
