@@ -672,26 +672,47 @@ __device__ __forceinline__ float lds_f1(const float* base, uint32_t off)   // ba
     return base[off >> 4];
 }
 
+// The first ids of a block's set, loaded before its size is known, so that the
+// wait for them overlaps the ones for the size and the particles' own data
+// (the table's rows are longer; what lies past the set is not used).  A block
+// waits for its staging chain with only one other block to fill the CU, and each
+// link counts: without this one the loop-end divergence sweep of 4.19 M
+// particles takes 180 us, with it 169.
+constexpr uint32_t kEarlyIds = 2048 / kBlock;
+struct SetIds {
+    uint32_t id[kEarlyIds];
+};
+
+__device__ __forceinline__ SetIds early_ids(const NbrLists& L, uint32_t b)
+{
+    static_assert(kEarlyIds * kBlock <= kStageCap, "ids past the block's row");
+    const uint32_t* g = L.stg + (size_t)b * kStageCap + threadIdx.x;
+    SetIds e;
+#pragma unroll
+    for (uint32_t u = 0; u < kEarlyIds; ++u) e.id[u] = g[u * kBlock];
+    return e;
+}
+
 // Loads an LDS-staged set: wr(k, ld(global id)) for k < count, then a block
 // barrier (reached by every thread).  Returns stage_n[b].  All of a thread's
-// index loads are issued first, then all its record loads (ld takes any valid
-// id: the lanes past the end load the set's last record), then the LDS
-// writes, so the loads of one thread are in flight together.
+// record loads are issued together (the lanes past the end load particle 0),
+// then the LDS writes.
 template <uint32_t CAP = kStageMax, class Ld, class Wr>
-__device__ __forceinline__ uint32_t stage_block(const NbrLists& L, uint32_t b, uint32_t sn, Ld&& ld, Wr&& wr)
+__device__ __forceinline__ uint32_t stage_block(const NbrLists& L, uint32_t b, uint32_t sn, const SetIds& early, Ld&& ld,
+                                                Wr&& wr)
 {
     using T = decltype(ld(0u));
     constexpr uint32_t U = (CAP + kBlock - 1) / kBlock;
     if (sn <= CAP && sn > 0u) {
-        const uint32_t* g = L.stg + (size_t)b * kStageCap;
+        const uint32_t* g = L.stg + (size_t)b * kStageCap + threadIdx.x;
         uint32_t gi[U];
         T d[U];
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u)
-            if (u * kBlock < sn) gi[u] = g[min(threadIdx.x + u * kBlock, sn - 1u)];
+        for (uint32_t u = kEarlyIds; u < U; ++u)
+            if (u * kBlock < sn) gi[u] = g[u * kBlock];
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u)
-            if (u * kBlock < sn) d[u] = ld(gi[u]);
+            if (u * kBlock < sn) d[u] = ld(threadIdx.x + u * kBlock < sn ? (u < kEarlyIds ? early.id[u] : gi[u]) : 0u);
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
             const uint32_t k = threadIdx.x + u * kBlock;
@@ -702,29 +723,38 @@ __device__ __forceinline__ uint32_t stage_block(const NbrLists& L, uint32_t b, u
     return sn;
 }
 
-template <class Ld, class Wr>
-__device__ __forceinline__ uint32_t stage_block(const NbrLists& L, uint32_t b, Ld&& ld, Wr&& wr)
-{
-    return stage_block(L, b, L.stage_n[b], ld, wr);
-}
-
-// The list counts and first two groups of particle i's fluid list (16-bit
-// when its block's set has them, else 32-bit) and boundary list, loaded
-// before the set is staged so that their latency hides behind it.
+// The list counts and first two groups of particle i's fluid list and boundary
+// list, loaded before the set is staged so that their latency hides behind
+// it.  The fluid groups are read without the counts (groups 0 and 1 exist for
+// every particle), the 16-bit ones whatever form the block's lists have.
 struct Head {
     uint32_t cnt;
     uint4 f0, f1, b0, b1;
 };
 
-__device__ __forceinline__ Head list_head(const NbrLists& L, uint32_t sn, uint32_t cap, uint32_t i)
+__device__ __forceinline__ Head list_head(const NbrLists& L, uint32_t cap, uint32_t i)
 {
-    const uint4* f = (sn != kUnstaged ? reinterpret_cast<const uint4*>(L.nbr16) : reinterpret_cast<const uint4*>(L.nbrf)) + i;
+    const uint4* f = reinterpret_cast<const uint4*>(L.nbr16) + i;
+    Head h;
+    h.cnt = L.cnt[i];
+    h.f0 = f[0];
+    h.f1 = f[cap];
+    return h;
+}
+
+// ... the rest of the head, once the counts and the set's size are there
+__device__ __forceinline__ void list_head_rest(const NbrLists& L, uint32_t sn, uint32_t cap, uint32_t i, Head& h)
+{
+    if (sn == kUnstaged) {
+        const uint4* f = reinterpret_cast<const uint4*>(L.nbrf) + i;
+        h.f0 = f[0];
+        h.f1 = f[cap];
+    }
     const uint4* bb = reinterpret_cast<const uint4*>(L.nbrb) + i;
-    const uint32_t cn = L.cnt[i];
-    const uint32_t nf = cn & 0xffffu, nb = cn >> 16;
-    const uint32_t f1 = sn != kUnstaged ? 8u : 4u;   // entries in group 0
+    const uint32_t nb = h.cnt >> 16;
     const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-    return Head{cn, nf > 0u ? f[0] : z, nf > f1 ? f[cap] : z, nb > 0u ? bb[0] : z, nb > 4u ? bb[cap] : z};
+    h.b0 = nb > 0u ? bb[0] : z;
+    h.b1 = nb > 4u ? bb[cap] : z;
 }
 
 // The fluid neighbors of particle i (block b, sn = stage_n[b]) in whichever

@@ -1112,11 +1112,13 @@ __global__ __launch_bounds__(kBlock, UM ? DFSPH_PV_WAVES : 1) void k_div_ws_init
     const uint32_t i = b * kBlock + threadIdx.x;
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
     const uint32_t sn0 = L.stage_n[b];
-    const Head hd = list_head(L, sn0, c.cap, ic);
+    const SetIds ids = early_ids(L, b);
+    Head hd = list_head(L, c.cap, ic);
     const float4 vi = vel_i[ic];
     const float4 pi = pos[ic];
     const float ki = ws_of(ic);
-    const uint32_t sn = stage_block<kStageMaxX>(L, b, sn0, [&](uint32_t g) {
+    list_head_rest(L, sn0, c.cap, ic, hd);
+    const uint32_t sn = stage_block<kStageMaxX>(L, b, sn0, ids, [&](uint32_t g) {
         const float4 v = vel_i[g];
         return PV{pos[g], make_float4(v.x, v.y, v.z, ws_of(g))};
     }, [&](uint32_t k, const PV& d) { st.put(k, d); });
@@ -1216,11 +1218,13 @@ __global__ __launch_bounds__(kBlock, UM ? DFSPH_PV_WAVES : 1) void k_div_source(
     const uint32_t i = b * kBlock + threadIdx.x;
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
     const uint32_t sn0 = L.stage_n[b];
-    const Head hd = list_head(L, sn0, c.cap, ic);
+    const SetIds ids = early_ids(L, b);
+    Head hd = list_head(L, c.cap, ic);
     const float4 pi = pos[ic];
     const float4 vi = vel[ic];
     const float ai = alpha[ic];
-    const uint32_t sn = stage_block<kStageMaxPV>(L, b, sn0, [&](uint32_t g) { return PV{pos[g], vel[g]}; },
+    list_head_rest(L, sn0, c.cap, ic, hd);
+    const uint32_t sn = stage_block<kStageMaxPV>(L, b, sn0, ids, [&](uint32_t g) { return PV{pos[g], vel[g]}; },
                                     [&](uint32_t k, const PV& d) { st.put(k, d); });
     float r = 0.0f;
     if (i < n && !is_source(L.rs, i)) r = radv[i];      // restricted out: stored value in the error sum
@@ -1274,11 +1278,12 @@ __global__ __launch_bounds__(kBlock) void k_jacobi(SimConst c, const DevTime* t,
     const uint32_t i = b * kBlock + threadIdx.x;
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
     const uint32_t sn0 = L.stage_n[b];
+    const SetIds ids = early_ids(L, b);
     const float ki = kk[ic];
     const float kv = DIV ? kappaV[ic] : 0.0f;
     const float4 pi = pos[ic];
     float4 v = vel[ic];
-    const uint32_t sn = stage_block(L, b, sn0, [&](uint32_t g) { return PK{pos[g], kk[g]}; },
+    const uint32_t sn = stage_block(L, b, sn0, ids, [&](uint32_t g) { return PK{pos[g], kk[g]}; },
                                     [&](uint32_t k, const PK& d) { st.put(k, d); });
     if (i >= n || !is_compute(L.rs, i)) return;
     if (DIV) kappaV[i] = kv + ki;
@@ -1329,10 +1334,12 @@ __global__ __launch_bounds__(kBlock, DFSPH_PV_WAVES) void k_xsph(SimConst c, con
     const uint32_t i = b * kBlock + threadIdx.x;
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
     const uint32_t sn0 = L.stage_n[b];
-    const Head hd = list_head(L, sn0, c.cap, ic);
+    const SetIds ids = early_ids(L, b);
+    Head hd = list_head(L, c.cap, ic);
     const float4 pi = pos[ic];
     const float4 vi = vel[ic];
-    const uint32_t sn = stage_block<kStageMaxX>(L, b, sn0, [&](uint32_t g) {
+    list_head_rest(L, sn0, c.cap, ic, hd);
+    const uint32_t sn = stage_block<kStageMaxX>(L, b, sn0, ids, [&](uint32_t g) {
         const float4 p = pos[g];
         const float4 v = vel[g];
         return PV{p, make_float4(v.x, v.y, v.z, p.w / rho[g])};
@@ -1451,11 +1458,12 @@ __global__ __launch_bounds__(kBlock) void k_pressure_ws(SimConst c, const DevTim
     const uint32_t i = b * kBlock + threadIdx.x;
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
     const uint32_t sn0 = L.stage_n[b];
+    const SetIds ids = early_ids(L, b);
     const float ki = ws_of(ic);
     const float4 pi = pos[ic];
     float4 v = vel[ic];
     const float4 aown = APPLY_ACC ? acc[ic] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const uint32_t sn = stage_block(L, b, sn0, [&](uint32_t g) { return PK{pos[g], ws_of(g)}; },
+    const uint32_t sn = stage_block(L, b, sn0, ids, [&](uint32_t g) { return PK{pos[g], ws_of(g)}; },
                                     [&](uint32_t k, const PK& d) { sP[k] = d.p; sK[k] = d.k; });
     if (i >= n || !is_compute(L.rs, i)) return;
     if (ktot) ktot[i] = ki;
@@ -1517,12 +1525,14 @@ __global__ __launch_bounds__(kBlock, UM ? DFSPH_PV_WAVES : 1) void k_density_sou
     const uint32_t i = b * kBlock + threadIdx.x;
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
     const uint32_t sn0 = L.stage_n[b];
-    const Head hd = list_head(L, sn0, c.cap, ic);
+    const SetIds ids = early_ids(L, b);
+    Head hd = list_head(L, c.cap, ic);
     const float4 pi = pos[ic];
     const float4 vi = vel[ic];
     const float a0 = alpha[ic], rho_i = rho[ic];
     const float kap0 = INIT ? 0.0f : kappa[ic];
-    const uint32_t sn = stage_block<kStageMaxPV>(L, b, sn0, [&](uint32_t g) { return PV{pos[g], vel[g]}; },
+    list_head_rest(L, sn0, c.cap, ic, hd);
+    const uint32_t sn = stage_block<kStageMaxPV>(L, b, sn0, ids, [&](uint32_t g) { return PV{pos[g], vel[g]}; },
                                     [&](uint32_t k, const PV& d) { st.put(k, d); });
     float r = 0.0f;
     if (i < n && !is_source(L.rs, i)) r = radv[i];      // restricted out: stored value in the error sum
@@ -1651,10 +1661,12 @@ __global__ __launch_bounds__(kBlock, UM ? DFSPH_PV_WAVES : 1) void k_features(Si
     const uint32_t i = b * kBlock + threadIdx.x;
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
     const uint32_t sn0 = L.stage_n[b];
-    const Head hd = list_head(L, sn0, c.cap, ic);
+    const SetIds ids = early_ids(L, b);
+    Head hd = list_head(L, c.cap, ic);
     const float4 pi = pos[ic];
     const float4 vi = vel[ic];
-    const uint32_t sn = stage_block<kStageMaxPV>(L, b, sn0, [&](uint32_t g) { return PV{pos[g], vel[g]}; },
+    list_head_rest(L, sn0, c.cap, ic, hd);
+    const uint32_t sn = stage_block<kStageMaxPV>(L, b, sn0, ids, [&](uint32_t g) { return PV{pos[g], vel[g]}; },
                                     [&](uint32_t k, const PV& d) { st.put(k, d); });
     if (i >= n) return;
     const uint32_t cn = hd.cnt;
