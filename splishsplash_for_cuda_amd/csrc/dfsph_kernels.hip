@@ -1436,7 +1436,9 @@ __global__ void k_update_vel(const DevTime* t, uint32_t n, const float4* acc, fl
 // kws holds the last solve's kappa increments.  No gate (unlike the divergence
 // warm start).  The applied k_i starts the particle's total of the step in
 // ktot (when given).
-template <int WS, bool APPLY_ACC, bool SOL>
+// With a uniform mass the stage is the Jacobi sweep's 16-byte records (52 KB, three
+// blocks per CU; 20-byte ones kept two: 203 us for 4.19 M particles, now 173).
+template <int WS, bool APPLY_ACC, bool SOL, bool UM>
 __global__ __launch_bounds__(kBlock) void k_pressure_ws(SimConst c, const DevTime* t, uint32_t n,
                                                         const float4* __restrict__ pos,
                                                         const float4* __restrict__ bpos, NbrLists L,
@@ -1445,8 +1447,7 @@ __global__ __launch_bounds__(kBlock) void k_pressure_ws(SimConst c, const DevTim
                                                         const float* __restrict__ kws, WsLearned lw, int rescale,
                                                         float* __restrict__ ktot)
 {
-    __shared__ float4 sP[kStageMax];
-    __shared__ float sK[kStageMax];
+    __shared__ PKStage<UM> st;
     const float ratio2 = rescale ? t->ratio2 : 1.0f;
     const float ihf2 = t->inv_h_future * t->inv_h_future;
     auto ws_of = [&](uint32_t j) -> float {
@@ -1464,7 +1465,7 @@ __global__ __launch_bounds__(kBlock) void k_pressure_ws(SimConst c, const DevTim
     float4 v = vel[ic];
     const float4 aown = APPLY_ACC ? acc[ic] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const uint32_t sn = stage_block(L, b, sn0, ids, [&](uint32_t g) { return PK{pos[g], ws_of(g)}; },
-                                    [&](uint32_t k, const PK& d) { sP[k] = d.p; sK[k] = d.k; });
+                                    [&](uint32_t k, const PK& d) { st.put(k, d); });
     if (i >= n || !is_compute(L.rs, i)) return;
     if (ktot) ktot[i] = ki;
     const uint32_t cn = L.cnt[i];
@@ -1477,7 +1478,7 @@ __global__ __launch_bounds__(kBlock) void k_pressure_ws(SimConst c, const DevTim
         const float s = keep(valid && kp.ok && fabsf(ks) > kEps, ks * pj.w * kp.g);
         ax += s * dx; ay += s * dy; az += s * dz;
     };
-    fluid_nbrs(L, c.cap, b, i, nf, sn, [&](uint32_t e) { return PK{lds_f4(sP, e), lds_f1(sK, e)}; },
+    fluid_nbrs(L, c.cap, b, i, nf, sn, [&](uint32_t e) { return st.get(e, c.m_uniform); },
                [&](uint32_t j) { return PK{pos[j], ws_of(j)}; },
                [&](const PK& d, bool valid) { fluid(d.p, d.k, valid); });
     if (fabsf(ki) > kEps) {
@@ -1970,7 +1971,9 @@ void launch_pressure_ws(hipStream_t s, int ws, bool apply_acc, const SimConst& c
     if (!n) return;
     const uint32_t g = nblk_xcd(n);
     const bool sol = L.sol.bvel != nullptr;
-#define PW(W, A, S) sweep_launch(k_pressure_ws<W, A, S>, g, s, c, t, n, pos, bpos, L, acc, vel, kws, lw, rescale, ktot)
+    const bool um = c.m_uniform > 0.0f;
+#define PWU(W, A, S, U) sweep_launch(k_pressure_ws<W, A, S, U>, g, s, c, t, n, pos, bpos, L, acc, vel, kws, lw, rescale, ktot)
+#define PW(W, A, S) do { if (um) PWU(W, A, S, true); else PWU(W, A, S, false); } while (0)
     if (ws == 1) {
         if (apply_acc) { if (sol) PW(1, true, true); else PW(1, true, false); }
         else { if (sol) PW(1, false, true); else PW(1, false, false); }
@@ -1979,6 +1982,7 @@ void launch_pressure_ws(hipStream_t s, int ws, bool apply_acc, const SimConst& c
         else { if (sol) PW(0, false, true); else PW(0, false, false); }
     }
 #undef PW
+#undef PWU
 }
 
 void launch_density_source(hipStream_t s, bool init, const SimConst& c, const DevTime* t, uint32_t n,
