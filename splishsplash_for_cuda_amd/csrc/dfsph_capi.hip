@@ -489,25 +489,35 @@ dfsph::CtlInit solve_ctl(Handle* h, bool div, uint32_t max_iter, double max_erro
 int jacobi_loop(Handle* h, bool div, uint32_t max_iter, double max_error, uint32_t* iters, double* err)
 {
     SolveCtl* sc = div ? &h->ctl->div : &h->ctl->dens;
+    // the step's total (applied warm start + increments) in kappaV h or kappa h_f^2
+    const dfsph::Totals fin = div ? dfsph::Totals{h->kapv[h->pc], h->kvtot[h->pc]}
+                                  : dfsph::Totals{h->kap[h->pc], h->ktot[h->pc]};
+    auto totals = [&]() -> int {
+        dfsph::launch_finish_totals(h->s, h->tm, h->n, div ? 0 : 1, fin);
+        HIPCHK(hipGetLastError());
+        return DFSPH_OK;
+    };
     const uint32_t min_iter = div ? h->p.min_iter_v : h->p.min_iter;
     (void)max_error;
+    // with min_iter == 0 the reference loop does not start (its error starts at 0)
+    const uint32_t first = std::min(min_iter, max_iter);
     if (h->n == 0 || max_iter == 0) {
         if (iters) *iters = 0;
         if (err) *err = 0.0;
-        return DFSPH_OK;
+        return totals();
     }
-    auto jacobi = [&]() -> int {
+    auto jacobi = [&](const dfsph::Totals& f) -> int {
         const int pr = pbeg(h, div ? DFSPH_KERNEL_DIV_JACOBI : DFSPH_KERNEL_DENS_JACOBI);
         if (div)
             dfsph::launch_jacobi(h->s, true, h->c, h->tm, h->n, h->pos[h->pc], h->bpos, lists(h), h->kk,
-                                 h->kapv[h->pc], h->vel[h->vc], sc);
+                                 h->kapv[h->pc], h->vel[h->vc], sc, f);
         else
             dfsph::launch_jacobi(h->s, false, h->c, h->tm, h->n, h->pos[h->pc], h->bpos, lists(h), h->kk,
-                                 nullptr, h->vel[h->vc], sc);
+                                 nullptr, h->vel[h->vc], sc, f);
         pend(h, pr);
         return pr;
     };
-    auto loop_end = [&]() {
+    auto loop_end = [&](uint32_t it) {      // of iteration it; its error is looked at from the minimum on
         const int pr = pbeg(h, div ? DFSPH_KERNEL_DIV_LOOP_END : DFSPH_KERNEL_DENS_LOOP_END);
         if (div)
             dfsph::launch_div_source(h->s, false, h->c, h->n, h->pos[h->pc], h->bpos, lists(h), h->vel[h->vc],
@@ -517,34 +527,35 @@ int jacobi_loop(Handle* h, bool div, uint32_t max_iter, double max_error, uint32
                                          h->vel[h->vc], h->rho, h->alpha, h->radv, h->kk, h->kap[h->pc], sc,
                                          h->partial);
         pend(h, pr);                    // the timed region is the sweep alone
-        dfsph::launch_solve_finalize(h->s, h->n, sc, h->partial, dfsph::Publish{h->ctl, h->tm, h->drec, ++h->seq});
+        if (it >= first)
+            dfsph::launch_solve_finalize(h->s, h->n, sc, h->partial, it,
+                                         dfsph::Publish{h->ctl, h->tm, h->drec, ++h->seq});
     };
     // The minimum iterations are always run.  After that, the velocity sweep
     // of the next iteration is queued before the host waits for the loop
     // state of the current one (published by the finalize kernel into host
     // memory), so the wait hides behind it; the source sweep is queued only
     // once the loop is known to continue.  The iteration count is exact, and
-    // at most one velocity sweep per solve exits at once.
-    // with min_iter == 0 the reference loop does not start (its error starts at 0)
-    const uint32_t first = std::min(min_iter, max_iter);
+    // at most one velocity sweep per solve finds the loop ended: it takes the
+    // step's totals.
     if (first == 0) {
         if (iters) *iters = 0;
         if (err) *err = 0.0;
-        return DFSPH_OK;
+        return totals();
     }
-    for (uint32_t k = 0; k < first; ++k) { jacobi(); loop_end(); }
+    for (uint32_t k = 1; k <= first; ++k) { jacobi(dfsph::Totals{}); loop_end(k); }
     uint32_t queued = first;
     SolveCtl res{};
     for (;;) {
         const bool spec = queued < max_iter;
-        const int pr = spec ? jacobi() : -1;
+        const int pr = spec ? jacobi(fin) : -1;
         HIPCHK(hipGetLastError());
         CHK(wait_record(h, h->seq));
         res = h->last.sc;
         if (res.done) pdrop(h, pr);   // that sweep exited at once
+        if (res.done && !spec) CHK(totals());
         if (res.done || !spec) break;
-        loop_end();
-        ++queued;
+        loop_end(++queued);
     }
     if (!res.done) return fail(DFSPH_ERR_STATE, "Jacobi loop ended without a decision");
     if (iters) *iters = res.iters;
@@ -606,9 +617,6 @@ int divergence_solve(Handle* h, uint32_t max_iter, double max_error, uint32_t* i
     CHK(jacobi_loop(h, true, max_iter, max_error, &it, err));
     if (iters) *iters = it;
     h->last_iters_v = it;
-    // the step's divergence total (applied warm start + increments) in kappaV h
-    dfsph::launch_finish_totals(h->s, h->tm, h->n, 0, h->kapv[h->pc], h->kvtot[h->pc]);
-    HIPCHK(hipGetLastError());
     return DFSPH_OK;
 }
 
@@ -670,8 +678,6 @@ int pressure_solve(Handle* h, uint32_t max_iter, double max_error, uint32_t* ite
     if (iters) *iters = it;
     h->last_iters = it;
     if (!h->p.enable_divergence) h->last_iters_v = 0;
-    // the step's density total (applied warm start + increments) in kappa h_f^2
-    dfsph::launch_finish_totals(h->s, h->tm, h->n, 1, h->kap[h->pc], h->ktot[h->pc]);
     if (h->mlp && dfsph::mlp_harvesting(h->mlp)) {
         // targets: what the reference warm start left to the iterations
         if (ws != DFSPH_WARMSTART_REFERENCE)
@@ -1183,7 +1189,7 @@ int dfsph_cfl(void* hv, double min_dt, double cfl_factor, double max_dt, double*
 {
     Handle* h = H(hv);
     if (!h->acc_valid) CHK(external_forces(h));
-    dfsph::launch_time_update(h->s, h->tm, 0.0, h->ctl, 1, cfl_factor, 2.0 * h->p.particle_radius, min_dt, max_dt, 0.0);
+    dfsph::launch_time_update(h->s, h->tm, 0.0, h->ctl, h->partial_f, h->n, 1, cfl_factor, 2.0 * h->p.particle_radius, min_dt, max_dt, 0.0);
     HIPCHK(hipGetLastError());
     if (!dt_out) return DFSPH_OK;       // stays on the device (dfsph_get_time reads it later)
     CHK(read_ctl(h));
@@ -1221,7 +1227,7 @@ int dfsph_update_time_step(void* hv, double h_future)
     Handle* h = H(hv);
     if (!(h_future > 0.0)) return fail(DFSPH_ERR_ARG, "time step must be positive");
     CHK(flush_vel(h));
-    dfsph::launch_time_update(h->s, h->tm, h_future, h->ctl, 0, 0, 0, 0, 0, 0);
+    dfsph::launch_time_update(h->s, h->tm, h_future, h->ctl, h->partial_f, h->n, 0, 0, 0, 0, 0, 0);
     HIPCHK(hipGetLastError());
     return DFSPH_OK;
 }
@@ -1336,7 +1342,7 @@ int dfsph_step(void* hv, dfsph_step_stats* st)
     CHK(external_forces(h));
     // h_future: CFL estimate, or the current step kept constant (the reference
     // takes TimeManager's step size, DFSPH_CUDA.cpp:299-306)
-    dfsph::launch_time_update(h->s, h->tm, 0.0, h->ctl, h->p.use_cfl ? 1 : 2, h->p.cfl_factor,
+    dfsph::launch_time_update(h->s, h->tm, 0.0, h->ctl, h->partial_f, h->n, h->p.use_cfl ? 1 : 2, h->p.cfl_factor,
                               2.0 * h->p.particle_radius, h->p.dt_min, h->p.dt_max, 0.0);
     h->pend_vel = true;
     const uint32_t seq0 = h->seq;

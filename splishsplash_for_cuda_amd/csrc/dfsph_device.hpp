@@ -138,6 +138,12 @@ __device__ __forceinline__ void ctl_init(const CtlInit& ci)
     s->ticket = 0;
 }
 
+// A solve's accumulated increments and the step totals they complete.
+struct Totals {
+    const float* inc;
+    float* tot;                    // nullptr: none to take
+};
+
 struct Publish {
     const DevCtl* dc;
     const DevTime* t;

@@ -79,16 +79,38 @@ __global__ void k_time_reset(DevTime* t, double h)
 
 // DFSPHCData::updateTimeStep (DFSPH_c_arrays_structure.cpp:1100-1106).  mode 0: the
 // given h_future; mode 1: the CFL estimate of cuda_CFL (DFSPH_core_cuda.cu:3380-3387),
-// h = cfl_factor * 0.4 * 2r / sqrt(max |v + a h|^2) clamped to [dt_min, dt_max];
-// mode 2: keep the current h (constant step, DFSPH_CUDA.cpp:302-306).
-__global__ void k_time_update(DevTime* t, double hf, const DevCtl* ctl, int mode,
-                              double cfl_factor, double diameter, double dt_min, double dt_max,
-                              double cfl_seed)
+// h = cfl_factor * 0.4 * 2r / sqrt(max |v + a h|^2) clamped to [dt_min, dt_max],
+// the maximum taken here from the XSPH sweep's nparts block maxima; mode 2: keep
+// the current h (constant step, DFSPH_CUDA.cpp:302-306).
+__global__ __launch_bounds__(kBlock) void k_time_update(DevTime* t, double hf, DevCtl* ctl, const float* partial,
+                                                        uint32_t nparts, int mode, double cfl_factor, double diameter,
+                                                        double dt_min, double dt_max, double cfl_seed)
 {
+    __shared__ float lds4[kBlock / 64];
+    if (mode == 1) {
+        constexpr uint32_t kBatch = 8;
+        float mm = 0.0f;
+        for (uint32_t k0 = threadIdx.x; k0 < nparts; k0 += kBatch * kBlock) {
+            float v[kBatch];
+#pragma unroll
+            for (uint32_t u = 0; u < kBatch; ++u) {
+                const uint32_t k = k0 + u * kBlock;
+                v[u] = k < nparts ? partial[k] : 0.0f;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kBatch; ++u) mm = fmaxf(mm, v[u]);
+        }
+        mm = wave_max(mm);
+        if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = mm;
+        __syncthreads();
+    }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (mode == 2) hf = t->hd;
         if (mode == 1) {
-            double m = (double)ctl->cfl_max;
+            float bm = lds4[0];
+            for (int k = 1; k < kBlock / 64; ++k) bm = fmaxf(bm, lds4[k]);
+            ctl->cfl_max = bm;
+            double m = (double)bm;
             m = m > cfl_seed ? m : cfl_seed;
             double h = cfl_factor * 0.4 * (diameter / sqrt(m));
             if (!(h < dt_max)) h = dt_max;
@@ -1044,8 +1066,11 @@ __device__ __forceinline__ void store_partial(double* partial, double bsum)
 // Sums the block partials in a fixed order (deterministic), forms
 // err = sum / N and evaluates the loop condition of cuda_divergenceSolve /
 // cuda_pressureSolve: continue while ((err > eta) || (it < min)) && (it < max).
+// it: the iterations made.  Below the minimum the loop continues whatever the
+// error, so only the iterations from the minimum on are followed by this kernel
+// (a launch and a one-block kernel, 4 to 6 us, three times less a step).
 __global__ __launch_bounds__(kBlock) void k_solve_finalize(SolveCtl* ctl, const double* partial, uint32_t nparts,
-                                                          Publish pub)
+                                                          uint32_t it, Publish pub)
 {
     __shared__ double lds4[kBlock / 64];
     if (!ctl->done) {
@@ -1067,7 +1092,6 @@ __global__ __launch_bounds__(kBlock) void k_solve_finalize(SolveCtl* ctl, const 
         const double tot = block_sum(acc, lds4);
         if (threadIdx.x == 0) {
             const double err = ctl->n_div > 0.0 ? tot / ctl->n_div : 0.0;
-            const uint32_t it = ctl->iters + 1;
             ctl->sum = tot;
             ctl->err = err;
             ctl->iters = it;
@@ -1262,20 +1286,39 @@ __global__ __launch_bounds__(kBlock, UM ? DFSPH_PV_WAVES : 1) void k_div_source(
     }
 }
 
+// End of a solve: the step's total = applied warm start + the solver's
+// accumulated increments, in dt-invariant units (scale h for kappaV, h_f^2 for kappa).
+__device__ __forceinline__ void finish_total(const DevTime& t, bool pressure, const Totals& f, uint32_t i)
+{
+    const float s = pressure ? t.h_future * t.h_future : t.h;
+    f.tot[i] = (f.tot[i] + f.inc[i]) * s;
+}
+
+__global__ void k_finish_totals(const DevTime* t, uint32_t n, int pressure, Totals f)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) finish_total(*t, pressure != 0, f, i);
+}
+
 // Jacobi velocity update: divergenceSolveParticle<false> (DFSPH_core_cuda.cu:400-481,
 // DIV: kappaV += k_i, step h) and pressureSolveParticle<false> (:867-951, step h_future):
 // v_i += step (sum_f [|k_i + k_j| > eps] (k_i + k_j) m_j gradW + [|k_i| > eps] sum_b k_i psi_j gradW)
+// The sweep queued before the loop's end is known (fin.tot given) takes the
+// step's totals instead of the iteration when the loop has ended.
 template <bool DIV, bool SOL, bool UM>
 __global__ __launch_bounds__(kBlock) void k_jacobi(SimConst c, const DevTime* t, uint32_t n,
                                                    const float4* __restrict__ pos,
                                                    const float4* __restrict__ bpos, NbrLists L,
                                                    const float* __restrict__ kk, float* __restrict__ kappaV,
-                                                   float4* __restrict__ vel, const SolveCtl* ctl)
+                                                   float4* __restrict__ vel, const SolveCtl* ctl, Totals fin)
 {
     __shared__ PKStage<UM> st;
-    if (ctl->done) return;
     const uint32_t b = xcd_block();
     const uint32_t i = b * kBlock + threadIdx.x;
+    if (ctl->done) {
+        if (fin.tot && i < n) finish_total(*t, !DIV, fin, i);
+        return;
+    }
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
     const uint32_t sn0 = L.stage_n[b];
     const SetIds ids = early_ids(L, b);
@@ -1321,7 +1364,8 @@ __global__ __launch_bounds__(kBlock) void k_jacobi(SimConst c, const DevTime* t,
 
 // DFSPH_viscosityXSPH_kernel (DFSPH_core_cuda.cu:1423-1510):
 // a_i = g - sum_f (1/h) nu (m_j / rho_j) (v_i - v_j) W_ij, fused with the CFL
-// maximum of |v + a h|^2 (DFSPH_CFLVelSquaredNorm_kernel, :3273-3278).
+// block maxima of |v + a h|^2 (DFSPH_CFLVelSquaredNorm_kernel, :3273-3278), which
+// k_time_update reduces.
 __global__ __launch_bounds__(kBlock, DFSPH_PV_WAVES) void k_xsph(SimConst c, const DevTime* t, uint32_t n,
                                                  const float4* __restrict__ pos, NbrLists L,
                                                  const float4* __restrict__ vel,
@@ -1330,6 +1374,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_PV_WAVES) void k_xsph(SimConst c, con
 {
     __shared__ float lds4[kBlock / 64];
     __shared__ PVSStage<true> st;                // (x, v, m / rho) of the staged set (the mass is not used)
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->escaped = 0;   // counted afresh by the step's update_pos
     const uint32_t b = xcd_block();
     const uint32_t i = b * kBlock + threadIdx.x;
     const uint32_t ic = i < n ? i : 0u;         // own loads before staging, so they overlap it
@@ -1383,33 +1428,6 @@ __global__ __launch_bounds__(kBlock, DFSPH_PV_WAVES) void k_xsph(SimConst c, con
         float bm = lds4[0];
         for (int k = 1; k < kBlock / 64; ++k) bm = fmaxf(bm, lds4[k]);
         partial[blockIdx.x] = bm;
-    }
-}
-
-// maximum of the XSPH kernel's block maxima (the CFL velocity bound)
-__global__ __launch_bounds__(kBlock) void k_cfl_finalize(DevCtl* ctl, const float* partial, uint32_t nparts)
-{
-    __shared__ float lds4[kBlock / 64];
-    constexpr uint32_t kBatch = 8;
-    float mm = 0.0f;
-    for (uint32_t k0 = threadIdx.x; k0 < nparts; k0 += kBatch * kBlock) {
-        float v[kBatch];
-#pragma unroll
-        for (uint32_t u = 0; u < kBatch; ++u) {
-            const uint32_t k = k0 + u * kBlock;
-            v[u] = k < nparts ? partial[k] : 0.0f;
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kBatch; ++u) mm = fmaxf(mm, v[u]);
-    }
-    mm = wave_max(mm);
-    if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = mm;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float bm = lds4[0];
-        for (int k = 1; k < kBlock / 64; ++k) bm = fmaxf(bm, lds4[k]);
-        ctl->cfl_max = bm;
-        ctl->escaped = 0;                      // counted afresh by the step's update_pos
     }
 }
 
@@ -1628,16 +1646,6 @@ __global__ void k_compact(uint32_t n, const uint32_t* keep, const uint32_t* rank
     copy_fluid(in, i, out, rank[i]);
 }
 
-// End of a solve: the step's total = applied warm start + the solver's
-// accumulated increments, in dt-invariant units (scale h for kappaV, h_f^2 for kappa).
-__global__ void k_finish_totals(const DevTime* t, uint32_t n, int pressure, const float* inc, float* tot)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float s = pressure ? t->h_future * t->h_future : t->h;
-    tot[i] = (tot[i] + inc[i]) * s;
-}
-
 // Features of the learned warm start, one neighbor sweep over the current state
 // (before the divergence warm start):
 //  0 rho / rho0 - 1            1 divergence source h / rho0 (unclamped)
@@ -1818,10 +1826,11 @@ void launch_nbr_ctl_init(hipStream_t s, DevCtl* c) { k_nbr_ctl_init<<<1, 64, 0, 
 
 void launch_time_reset(hipStream_t s, DevTime* t, double h) { k_time_reset<<<1, 64, 0, s>>>(t, h); }
 
-void launch_time_update(hipStream_t s, DevTime* t, double hf, const DevCtl* ctl, int mode,
+void launch_time_update(hipStream_t s, DevTime* t, double hf, DevCtl* ctl, const float* partial, uint32_t n, int mode,
                         double cfl_factor, double diameter, double dt_min, double dt_max, double seed)
 {
-    k_time_update<<<1, 64, 0, s>>>(t, hf, ctl, mode, cfl_factor, diameter, dt_min, dt_max, seed);
+    k_time_update<<<1, kBlock, 0, s>>>(t, hf, ctl, partial, nblk_xcd(n ? n : 1), mode, cfl_factor, diameter, dt_min,
+                                       dt_max, seed);
 }
 
 void launch_time_step_end(hipStream_t s, DevTime* t, const Publish& pub) { k_time_step_end<<<1, 64, 0, s>>>(t, pub); }
@@ -1927,20 +1936,21 @@ void launch_div_source(hipStream_t s, bool init, const SimConst& c, uint32_t n, 
 #undef DS
 }
 
-void launch_solve_finalize(hipStream_t s, uint32_t n, SolveCtl* ctl, const double* partial, const Publish& pub)
+void launch_solve_finalize(hipStream_t s, uint32_t n, SolveCtl* ctl, const double* partial, uint32_t it,
+                           const Publish& pub)
 {
-    k_solve_finalize<<<1, kBlock, 0, s>>>(ctl, partial, nblk_xcd(n ? n : 1), pub);
+    k_solve_finalize<<<1, kBlock, 0, s>>>(ctl, partial, nblk_xcd(n ? n : 1), it, pub);
 }
 
 void launch_jacobi(hipStream_t s, bool div, const SimConst& c, const DevTime* t, uint32_t n, const float4* pos,
                    const float4* bpos, const NbrLists& L, const float* kk, float* kappaV,
-                   float4* vel, const SolveCtl* ctl)
+                   float4* vel, const SolveCtl* ctl, const Totals& fin)
 {
     if (!n) return;
     const uint32_t g = nblk_xcd(n);
     const bool sol = L.sol.bvel != nullptr;
     const bool um = c.m_uniform > 0.0f;
-#define JA(D, S, U) sweep_launch(k_jacobi<D, S, U>, g, s, c, t, n, pos, bpos, L, kk, kappaV, vel, ctl)
+#define JA(D, S, U) sweep_launch(k_jacobi<D, S, U>, g, s, c, t, n, pos, bpos, L, kk, kappaV, vel, ctl, fin)
 #define JAU(D, S) do { if (um) JA(D, S, true); else JA(D, S, false); } while (0)
     if (div) { if (sol) JAU(true, true); else JAU(true, false); }
     else { if (sol) JAU(false, true); else JAU(false, false); }
@@ -1954,7 +1964,6 @@ void launch_xsph(hipStream_t s, const SimConst& c, const DevTime* t, uint32_t n,
 {
     const uint32_t g = nblk_xcd(n ? n : 1);
     sweep_launch(k_xsph, g, s, c, t, n, pos, L, vel, rho, acc, ctl, partial);
-    k_cfl_finalize<<<1, kBlock, 0, s>>>(ctl, partial, g);
 }
 
 void launch_update_vel(hipStream_t s, const DevTime* t, uint32_t n, const float4* acc, float4* vel, float* kappa,
@@ -2026,9 +2035,9 @@ void launch_compact(hipStream_t s, uint32_t n, const uint32_t* keep, const uint3
     if (n) k_compact<<<nblk(n), kBlock, 0, s>>>(n, keep, rank, in, out);
 }
 
-void launch_finish_totals(hipStream_t s, const DevTime* t, uint32_t n, int pressure, const float* inc, float* tot)
+void launch_finish_totals(hipStream_t s, const DevTime* t, uint32_t n, int pressure, const Totals& f)
 {
-    if (n) k_finish_totals<<<nblk(n), kBlock, 0, s>>>(t, n, pressure, inc, tot);
+    if (n) k_finish_totals<<<nblk(n), kBlock, 0, s>>>(t, n, pressure, f);
 }
 
 void launch_features(hipStream_t s, const SimConst& c, const DevTime* t, uint32_t n, const float4* pos,

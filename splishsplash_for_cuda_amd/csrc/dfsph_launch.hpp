@@ -28,7 +28,7 @@ void launch_exclusive_scan(hipStream_t s, uint32_t* in, uint32_t* out, uint32_t 
 
 void launch_nbr_ctl_init(hipStream_t s, DevCtl* c);
 void launch_time_reset(hipStream_t s, DevTime* t, double h);
-void launch_time_update(hipStream_t s, DevTime* t, double hf, const DevCtl* ctl, int mode,
+void launch_time_update(hipStream_t s, DevTime* t, double hf, DevCtl* ctl, const float* partial, uint32_t n, int mode,
                         double cfl_factor, double diameter, double dt_min, double dt_max, double seed);
 void launch_time_step_end(hipStream_t s, DevTime* t, const Publish& pub = Publish{});
 void launch_time_set(hipStream_t s, DevTime* t, double h, double hp, double time);
@@ -72,10 +72,11 @@ void launch_div_source(hipStream_t s, bool init, const SimConst& c, uint32_t n, 
                        const float* alpha, float* radv, float* kk, float* kappaV, SolveCtl* ctl, double* partial,
                        const CtlInit& ci = CtlInit{});
 // the one-block error reduction and loop decision after a loop-end sweep of n particles
-void launch_solve_finalize(hipStream_t s, uint32_t n, SolveCtl* ctl, const double* partial, const Publish& pub);
+void launch_solve_finalize(hipStream_t s, uint32_t n, SolveCtl* ctl, const double* partial, uint32_t it,
+                           const Publish& pub);
 void launch_jacobi(hipStream_t s, bool div, const SimConst& c, const DevTime* t, uint32_t n, const float4* pos,
                    const float4* bpos, const NbrLists& L, const float* kk, float* kappaV,
-                   float4* vel, const SolveCtl* ctl);
+                   float4* vel, const SolveCtl* ctl, const Totals& fin);
 void launch_xsph(hipStream_t s, const SimConst& c, const DevTime* t, uint32_t n, const float4* pos,
                  const NbrLists& L, const float4* vel, const float* rho, float4* acc,
                  DevCtl* ctl, float* partial);
@@ -96,7 +97,7 @@ void launch_keep_inside(hipStream_t s, uint32_t n, const float4* pos, const floa
 void launch_keep_from_u8(hipStream_t s, uint32_t n, const uint8_t* k8, uint32_t* keep);
 void launch_compact(hipStream_t s, uint32_t n, const uint32_t* keep, const uint32_t* rank, const FluidPtrs& in,
                     const FluidPtrs& out);
-void launch_finish_totals(hipStream_t s, const DevTime* t, uint32_t n, int pressure, const float* inc, float* tot);
+void launch_finish_totals(hipStream_t s, const DevTime* t, uint32_t n, int pressure, const Totals& f);
 // features of the learned warm start; also copies the last step's totals
 // (ktot, kvtot) into prev_p, prev_v for the sweeps' bound
 void launch_features(hipStream_t s, const SimConst& c, const DevTime* t, uint32_t n, const float4* pos,
