@@ -756,7 +756,7 @@ int alloc_fluid(Handle* h, uint32_t cap)
     // neighbor sets: one per block of the XCD-padded grid
     const uint32_t nblocks = dfsph::grid_blocks_xcd(cap);
     CHK(dalloc(h->stage_n, nblocks));
-    CHK(dalloc(h->nbr_part, 2 * (size_t)nblocks));
+    CHK(dalloc(h->nbr_part, 2 * (size_t)std::max(nblocks, 2u * dfsph::kNumCu)));   // (a split search: at most kNumCu)
     CHK(dalloc(h->stg, (size_t)nblocks * dfsph::kStageCap));
     CHK(ensure_tmp(h, std::max(cap, h->nb)));
     CHK(ensure_partials(h, cap));

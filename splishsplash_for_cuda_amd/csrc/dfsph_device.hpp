@@ -37,6 +37,7 @@ namespace dfsph {
 constexpr int kBlock = DFSPH_BLOCK;
 static_assert(kBlock == 256 || kBlock == 512, "256 or 512 threads: 4 or 8 wavefronts of 64");
 constexpr int kNumXcd = 8;         // MI355X: 8 XCDs, blocks dispatched round robin
+constexpr uint32_t kNumCu = 256;
 constexpr float kEps = 1.0e-5f;    // m_eps (DFSPH_define_cuda.h:7)
 
 // Constants of one simulation, passed by value to every kernel.

@@ -543,7 +543,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
                                                       uint16_t* __restrict__ nbr16, uint32_t* __restrict__ nbrf,
                                                       uint32_t* __restrict__ nbrb, uint32_t* __restrict__ cnt,
                                                       uint32_t* __restrict__ stage_n, uint32_t* __restrict__ stg,
-                                                      Restrict rs, uint4* __restrict__ part)
+                                                      Restrict rs, uint4* __restrict__ part, uint32_t split)
 {
     // The tables under construction lie in the first half of the staged
     // positions and are dead once those are loaded.
@@ -562,9 +562,11 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
     static_assert((kStageCap - 1) * 16 <= 0xffffu && kBigCells < 0xffffu, "16-bit byte offsets / cell ids");
     uint32_t* s_wu = reinterpret_cast<uint32_t*>(s_w);
 
-    const uint32_t b = xcd_block();
+    // split blocks build the same set, each searches its share of the wavefronts
+    const uint32_t b = xcd_block() / split, share = xcd_block() % split;
     const uint32_t i = b * kBlock + threadIdx.x;
     const bool act = i < n;
+    const bool mine = (threadIdx.x >> 6) / (kBlock / 64u / split) == share;
     float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     int cx = 0, cy = 0, cz = 0;
     if (act) {
@@ -698,7 +700,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
                 if (threadIdx.x == 0) { s_off[U] = tot; s_boff[U] = Sb; }
                 S = tot <= c.stage_cap ? tot : kUnstaged;
                 // each lane's rows (dy, dz) as (first, last) set cell of x-1..x+1
-                if (act) {
+                if (act && mine) {
 #pragma unroll
                     for (int r = 0; r < 9; ++r) {
                         const int y = cy + r / 3 - 1, z = cz + r % 3 - 1;
@@ -717,7 +719,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
     const uint32_t room = U <= kSetCells ? kNbrStage : kHalfStage;
     const bool lds_search = S <= room && c.stage_lds > 0u;
     const bool lds_bnd = lds_search && S + Sb <= room;        // boundary staged at [S, S + Sb)
-    if (threadIdx.x == 0) stage_n[b] = S == kUnstaged || S <= c.stage_lds ? S : (S | kSetNoLds);
+    if (threadIdx.x == 0 && share == 0u) stage_n[b] = S == kUnstaged || S <= c.stage_lds ? S : (S | kSetNoLds);
     if (S != kUnstaged) {
         // eight lanes per set cell: its particles' ids and positions to their set places
         uint32_t* g_out = stg + (size_t)b * kStageCap;
@@ -726,7 +728,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
             const uint32_t off = s_off[u], e = s_off[u + 1u], g0 = s_src[u];
             for (uint32_t k = off + sub; k < e; k += 8u) {
                 if (lds_search) st.put(k, pos[g0 + k]);
-                g_out[k] = g0 + k;
+                if (share == 0u) g_out[k] = g0 + k;
             }
             if (lds_bnd) {
                 const uint32_t boff = s_boff[u], be = s_boff[u + 1u], j0 = s_bs[u];
@@ -736,8 +738,8 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
         __syncthreads();
     }
     uint32_t total = 0, trunc = 0, stored_f = 0, stored_b = 0, stored_u32 = 0;
-    if (act && !is_source(rs, i)) cnt[i] = 0;           // restricted out: no lists
-    if (act && is_source(rs, i)) {
+    if (act && mine && !is_source(rs, i)) cnt[i] = 0;   // restricted out: no lists
+    if (act && mine && is_source(rs, i)) {
         const uint32_t maxn = c.max_nbr, cap = c.cap;
         const float hk2 = c.hk2;
         uint32_t nf = 0, nb = 0;                 // found; stored while below max_neighbors
@@ -860,7 +862,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
         stored_b = sb;
         stored_u32 = S == kUnstaged ? sf : 0u;
     }
-    // the block's statistics go to part[2b], part[2b + 1] (k_nbr_finalize
+    // the block's statistics go to its two records in part (k_nbr_finalize
     // sums them): per-wave atomics on one control line would serialise
     const uint32_t wv[5] = {(uint32_t)wave_max_i((int)total), wave_total_u(trunc), wave_total_u(stored_f),
                             wave_total_u(stored_b), wave_total_u(stored_u32)};
@@ -875,9 +877,9 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
                 const uint32_t x = (uint32_t)s_w[5 * v + k];
                 a[k] = k == 0 ? max(a[0], x) : a[k] + x;
             }
-        const uint32_t unstaged = S > c.stage_lds && n > b * kBlock ? 1u : 0u;
-        part[2 * b] = make_uint4(a[0], a[1], a[2], a[3]);
-        part[2 * b + 1] = make_uint4(a[4], unstaged, 0u, 0u);
+        const uint32_t unstaged = S > c.stage_lds && n > b * kBlock && share == 0u ? 1u : 0u;
+        part[2 * xcd_block()] = make_uint4(a[0], a[1], a[2], a[3]);
+        part[2 * xcd_block() + 1] = make_uint4(a[4], unstaged, 0u, 0u);
     }
 }
 
@@ -1762,6 +1764,18 @@ static inline uint32_t nblk_xcd(uint32_t n)
 
 uint32_t grid_blocks_xcd(uint32_t n) { return nblk_xcd(n ? n : 1); }
 
+// Blocks that share a set in the search of n particles: as long as the blocks
+// leave CUs idle, the candidate tests and list writing of a block's wavefronts
+// (most of its time, at the rate of its CU's vector units) go to several, each
+// with its own copy of the set.  16k particles: 39 us with one, 37 with eight
+// (a step 333 -> 317 us); 1600 particles: a step 289 -> 284 us.
+uint32_t search_split(uint32_t n)
+{
+    uint32_t split = 1;
+    while (split < kBlock / 64u && nblk(n) * split * 2u <= kNumCu) split *= 2u;
+    return split;
+}
+
 static thread_local hipEvent_t tl_ev_start = nullptr, tl_ev_stop = nullptr;
 
 void arm_sweep_events(hipEvent_t start, hipEvent_t stop)
@@ -1876,13 +1890,13 @@ void launch_neighbors(hipStream_t s, const SimConst& c, bool indirect, const flo
                       const Restrict& rs, uint4* part, DevCtl* ctl)
 {
     if (!n) return;
-    const uint32_t g = nblk_xcd(n);
+    const uint32_t split = search_split(n), g = nblk_xcd(n) * split;
     if (indirect)
         k_neighbors<true><<<g, kBlock, 0, s>>>(c, pos, cs_f, perm, bpos, cs_b, n, nbr16, nbrf, nbrb, cnt, stage_n, stg,
-                                               rs, part);
+                                               rs, part, split);
     else
         k_neighbors<false><<<g, kBlock, 0, s>>>(c, pos, cs_f, perm, bpos, cs_b, n, nbr16, nbrf, nbrb, cnt, stage_n, stg,
-                                                rs, part);
+                                                rs, part, split);
     k_nbr_finalize<<<1, kBlock, 0, s>>>(part, g, ctl);
 }
 

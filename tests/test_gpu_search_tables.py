@@ -138,3 +138,23 @@ def test_sweeps_agree_between_list_forms(name):
     for other in out[1:]:
         for a, b in zip(out[0], other):
             assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("blocks", [32, 33, 65, 129])
+def test_search_shares(blocks):
+    """Blocks that share a set (8, 4, 2 and 1 of them): one particle in the last one,
+    lists as the search without sets has them, neighbors as a k-d tree counts them."""
+    from scipy.spatial import cKDTree
+    n = 512 * (blocks - 1) + 1
+    rng = np.random.default_rng(blocks)
+    x = _jitter(fluid_block((0.05, 0.05, 0.05), (38, 38, -(-n // 1444)), 2 * R), rng, 0.2)[:n].astype(np.float32)
+    walls = box_surface((0, 0, 0), (2.0, 2.0, 0.2 + 2 * R * -(-n // 1444)), 2 * R).astype(np.float32)
+    pos, bpos, nf, nb, L, stats = _search(x, walls, 96, S.LISTS_AUTO)
+    _, _, gf, gb, G, gstats = _search(x, walls, 96, S.LISTS_GLOBAL)
+    assert len(pos) == n and stats == gstats
+    assert np.array_equal(nf, gf) and np.array_equal(nb, gb) and np.array_equal(L, G)
+    p = cKDTree(pos.astype(np.float64))
+    for r, low in ((H * (1 - 1e-5), True), (H * (1 + 1e-5), False)):
+        wf = p.query_ball_point(pos.astype(np.float64), r, return_length=True) - 1
+        wb = cKDTree(bpos.astype(np.float64)).query_ball_point(pos.astype(np.float64), r, return_length=True)
+        assert ((wf <= nf) & (wb <= nb)).all() if low else ((wf >= nf) & (wb >= nb)).all()
