@@ -321,7 +321,8 @@ dfsph::Restrict restriction(const Handle* h)
 dfsph::NbrLists lists(const Handle* h)
 {
     const dfsph::Solids sol{h->ns ? h->bvel : nullptr, h->sforce, h->fscale};
-    return dfsph::NbrLists{h->nbr16, h->nbrf, h->nbrb, h->cnt, h->stage_n, h->stg, restriction(h), sol};
+    return dfsph::NbrLists{h->nbr16, h->nbrf, h->nbrb, h->cnt, h->stage_n, h->stg, restriction(h), sol,
+                           dfsph::list_stream(h->n)};
 }
 
 int ensure_scan(Handle* h, uint32_t n)

@@ -300,6 +300,9 @@ struct Solids {
     float fscale;
 };
 
+// parts of the lists that a sweep reads past the caches (list_stream() says when)
+enum : uint32_t { kStreamLists = 1u, kStreamIds = 2u };
+
 struct NbrLists {
     const uint16_t* nbr16;         // 16-bit fluid lists (blocks with a staged set)
     const uint32_t* nbrf;          // 32-bit fluid lists (unstaged blocks)
@@ -309,6 +312,7 @@ struct NbrLists {
     const uint32_t* stg;           // per block: global ids of the set (kStageCap each)
     Restrict rs;                   // solver restriction (mode 0: none)
     Solids sol;
+    uint32_t stream;               // kStreamLists, kStreamIds: read non-temporally
 };
 
 // boundary neighbor record of the sweeps: position + psi, velocity + solid index
@@ -557,6 +561,18 @@ __device__ __forceinline__ void for_each_adjacent_range(const SimConst& c, int c
     }
 }
 
+// group of 8 entries of the 16-bit lists
+__device__ __forceinline__ uint4 list16_group(const NbrLists& L, size_t at)
+{
+    const uint4* p = reinterpret_cast<const uint4*>(L.nbr16) + at;
+    if (L.stream & kStreamLists) {
+        typedef uint32_t V __attribute__((ext_vector_type(4)));
+        const V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+        return make_uint4(v[0], v[1], v[2], v[3]);
+    }
+    return *p;
+}
+
 // Neighbor loops with memory-level parallelism: a batch of 8 list entries is
 // one 16-byte load (16-bit lists) or two (32-bit lists) per lane, then the 8
 // neighbors' gathers can all be in flight before the first one is used.  Entries
@@ -569,7 +585,9 @@ __device__ __forceinline__ void for_each_adjacent_range(const SimConst& c, int c
 // Each batch first issues the loads of all its neighbors (load(entry) returns
 // the neighbor's data), then runs body(data, valid) on them, so the LDS or
 // L2 latency of one neighbor overlaps the others'; the next batch's list
-// group is loaded while the current batch computes.
+// group is loaded while the current batch computes: issued before it, which
+// the scheduling barrier keeps so (it sank to the batch's end; 1.05 M particles:
+// Jacobi 50.4 -> 46.5 us, density warm start 49.2 -> 44).
 // 16-bit lists: the batches that are full in every lane of the wave run
 // unmasked, then half batches of 4 until the longest list ends.  With whole
 // partial batches after the full ones a wave of 28 to 33 neighbors ran 40 slots,
@@ -577,12 +595,11 @@ __device__ __forceinline__ void for_each_adjacent_range(const SimConst& c, int c
 // other sweeps, which wait for their staging, 1 to 4 %.  (The same split of
 // the 32-bit lists made the sweeps with many wall neighbors 15 % slower.)
 template <class Load, class Body>
-__device__ __forceinline__ void for_each_nbr16(const uint16_t* __restrict__ lists, uint32_t cap, uint32_t i,
+__device__ __forceinline__ void for_each_nbr16(const NbrLists& L, uint32_t cap, uint32_t i,
                                                uint32_t count, uint4 q, uint4 qn, Load&& load, Body&& body)
 {
     // q, qn: the particle's groups 0 and 1 (loaded by the caller)
     using T = decltype(load(0u));
-    const uint4* p = reinterpret_cast<const uint4*>(lists) + i;
     uint32_t k = 0;
     // batches that are full in every lane: no masking
     uint32_t full = 0;
@@ -590,7 +607,8 @@ __device__ __forceinline__ void for_each_nbr16(const uint16_t* __restrict__ list
     for (; k < full; k += 8u) {
         const uint32_t w[4] = {q.x, q.y, q.z, q.w};
         q = qn;
-        if (k + 16u < count) qn = p[(size_t)((k >> 3) + 2) * cap];   // two groups ahead, when a batch reads it
+        if (k + 16u < count) qn = list16_group(L, i + (size_t)((k >> 3) + 2) * cap);   // two ahead, when read
+        __builtin_amdgcn_sched_barrier(0);
         T it[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) it[u] = load((w[u >> 1] >> ((u & 1) * 16)) & 0xffffu);
@@ -607,20 +625,22 @@ __device__ __forceinline__ void for_each_nbr16(const uint16_t* __restrict__ list
         for (int u = 0; u < 4; ++u) body(it[u], at + u < count);
     };
     for (; k < count; k += 8u) {
-        half(q.x, q.y, k);
-        if (k + 4u < count) half(q.z, q.w, k + 4u);
+        const uint4 w = q;
         q = qn;
-        if (k + 16u < count) qn = p[(size_t)((k >> 3) + 2) * cap];
+        if (k + 16u < count) qn = list16_group(L, i + (size_t)((k >> 3) + 2) * cap);
+        __builtin_amdgcn_sched_barrier(0);
+        half(w.x, w.y, k);
+        if (k + 4u < count) half(w.z, w.w, k + 4u);
     }
 }
 
 template <class Load, class Body>
-__device__ __forceinline__ void for_each_nbr16(const uint16_t* __restrict__ lists, uint32_t cap, uint32_t i,
+__device__ __forceinline__ void for_each_nbr16(const NbrLists& L, uint32_t cap, uint32_t i,
                                                uint32_t count, Load&& load, Body&& body)
 {
-    const uint4* p = reinterpret_cast<const uint4*>(lists) + i;
     const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-    for_each_nbr16(lists, cap, i, count, count > 0u ? p[0] : z, count > 8u ? p[cap] : z, load, body);
+    for_each_nbr16(L, cap, i, count, count > 0u ? list16_group(L, i) : z,
+                   count > 8u ? list16_group(L, i + (size_t)cap) : z, load, body);
 }
 
 template <class Load, class Body>
@@ -667,10 +687,10 @@ __device__ __forceinline__ void for_each_nbr32(const uint32_t* __restrict__ list
 
 // the plain forms: f(entry, valid)
 template <class F>
-__device__ __forceinline__ void for_each_nbr16(const uint16_t* __restrict__ lists, uint32_t cap, uint32_t i,
+__device__ __forceinline__ void for_each_nbr16(const NbrLists& L, uint32_t cap, uint32_t i,
                                                uint32_t count, F&& f)
 {
-    for_each_nbr16(lists, cap, i, count, [](uint32_t e) { return e; }, f);
+    for_each_nbr16(L, cap, i, count, [](uint32_t e) { return e; }, f);
 }
 
 template <class F>
@@ -708,8 +728,15 @@ __device__ __forceinline__ SetIds early_ids(const NbrLists& L, uint32_t b)
     static_assert(kEarlyIds * kBlock <= kStageCap, "ids past the block's row");
     const uint32_t* g = L.stg + (size_t)b * kStageCap + threadIdx.x;
     SetIds e;
+    if (L.stream & kStreamIds) {
+        asm volatile("");                       // the branches' loads are not to be merged
 #pragma unroll
-    for (uint32_t u = 0; u < kEarlyIds; ++u) e.id[u] = g[u * kBlock];
+        for (uint32_t u = 0; u < kEarlyIds; ++u) e.id[u] = __builtin_nontemporal_load(g + u * kBlock);
+        asm volatile("");
+    } else {
+#pragma unroll
+        for (uint32_t u = 0; u < kEarlyIds; ++u) e.id[u] = g[u * kBlock];
+    }
     return e;
 }
 
@@ -754,11 +781,10 @@ struct Head {
 
 __device__ __forceinline__ Head list_head(const NbrLists& L, uint32_t cap, uint32_t i)
 {
-    const uint4* f = reinterpret_cast<const uint4*>(L.nbr16) + i;
     Head h;
     h.cnt = L.cnt[i];
-    h.f0 = f[0];
-    h.f1 = f[cap];
+    h.f0 = list16_group(L, i);
+    h.f1 = list16_group(L, i + (size_t)cap);
     return h;
 }
 
@@ -786,10 +812,10 @@ __device__ __forceinline__ void fluid_nbrs(const NbrLists& L, uint32_t cap, uint
                                            uint32_t sn, FL&& lds, FG&& glob, Body&& body)
 {
     if (sn <= CAP) {
-        for_each_nbr16(L.nbr16, cap, i, nf, lds, body);
+        for_each_nbr16(L, cap, i, nf, lds, body);
     } else if (sn != kUnstaged) {
         const uint32_t* g = L.stg + (size_t)b * kStageCap;
-        for_each_nbr16(L.nbr16, cap, i, nf, [&](uint32_t e) { return glob(g[e >> 4]); }, body);
+        for_each_nbr16(L, cap, i, nf, [&](uint32_t e) { return glob(g[e >> 4]); }, body);
     } else {
         for_each_nbr32(L.nbrf, cap, i, nf, i, glob, body);
     }
@@ -802,10 +828,10 @@ __device__ __forceinline__ void fluid_nbrs(const NbrLists& L, uint32_t cap, uint
 {
     const uint32_t nf = hd.cnt & 0xffffu;
     if (sn <= CAP) {
-        for_each_nbr16(L.nbr16, cap, i, nf, hd.f0, hd.f1, lds, body);
+        for_each_nbr16(L, cap, i, nf, hd.f0, hd.f1, lds, body);
     } else if (sn != kUnstaged) {
         const uint32_t* g = L.stg + (size_t)b * kStageCap;
-        for_each_nbr16(L.nbr16, cap, i, nf, hd.f0, hd.f1, [&](uint32_t e) { return glob(g[e >> 4]); }, body);
+        for_each_nbr16(L, cap, i, nf, hd.f0, hd.f1, [&](uint32_t e) { return glob(g[e >> 4]); }, body);
     } else {
         for_each_nbr32(L.nbrf, cap, i, nf, i, hd.f0, hd.f1, glob, body);
     }

@@ -1776,6 +1776,22 @@ uint32_t search_split(uint32_t n)
     return split;
 }
 
+// What the sweeps over n particles read past the caches (non-temporal loads).
+// A pass reads some 128 bytes a particle, half of them its list, and the passes
+// of a step read the same lists again: up to the 256 MB of the memory-side
+// cache they stay there, and streaming them costs 5 % (1.05 M: Jacobi 50.4 -> 52
+// us).  Beyond, the lists only drive out the records the blocks' sets are gathered
+// from.  Lists streamed, divergence Jacobi: 1.57 M 51.3 -> 52.8 us, 1.84 M 64.2
+// -> 61.5 (but loop end 73.5 -> 75.5), 2.1 M 76.1 -> 68.7, 3.1 M 117 -> 100, 4.2 M
+// 157 -> 137, 6.6 M 234 -> 216.  The sets' ids with them: 2.1 M 68.7 -> 70.7, 3.1 M
+// even, 4.2 M 137 -> 130, 6.6 M 216 -> 210.
+uint32_t list_stream(uint32_t n)
+{
+    constexpr uint32_t kPassBytes = 128u, kCacheBytes = 1u << 28;
+    if (n < kCacheBytes / kPassBytes) return 0u;
+    return n < 2u * (kCacheBytes / kPassBytes) ? kStreamLists : kStreamLists | kStreamIds;
+}
+
 static thread_local hipEvent_t tl_ev_start = nullptr, tl_ev_stop = nullptr;
 
 void arm_sweep_events(hipEvent_t start, hipEvent_t stop)

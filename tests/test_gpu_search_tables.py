@@ -158,3 +158,28 @@ def test_search_shares(blocks):
         wf = p.query_ball_point(pos.astype(np.float64), r, return_length=True) - 1
         wb = cKDTree(bpos.astype(np.float64)).query_ball_point(pos.astype(np.float64), r, return_length=True)
         assert ((wf <= nf) & (wb <= nb)).all() if low else ((wf >= nf) & (wb >= nb)).all()
+
+
+@pytest.mark.parametrize("n", [(1 << 21) - 1, 1 << 21, 1 << 22])
+def test_streamed_lists(n):
+    """Sweeps on both sides of the sizes from which the lists, then the sets' ids, are
+    read past the caches: the same bits as over the 32-bit lists, which never are."""
+    rng = np.random.default_rng(n)
+    x = fluid_block((0.05, 0.05, 0.05), (128, 128, -(-n // 16384)), 2 * R)[:n].astype(np.float32)
+    x += rng.uniform(-0.2 * R, 0.2 * R, x.shape).astype(np.float32)
+    v = rng.normal(scale=0.3, size=x.shape).astype(np.float32)
+    walls = box_surface((0, 0, 0), (6.6, 6.6, 0.2 + 2 * R * -(-n // 16384)), 2 * R).astype(np.float32)
+    out = []
+    for mode in (S.LISTS_AUTO, S.LISTS_GLOBAL):
+        s = S.Solver(S.default_params(particle_radius=R, max_neighbors=60, list_mode=mode))
+        s.upload_boundary(walls)
+        s.upload_fluid(x, v)
+        s.neighbor_search()
+        s.divergence_solve(2, 0.0)
+        s.external_forces()
+        s.update_vel()
+        s.pressure_solve(2, 0.0)
+        out.append([s.download(f) for f in (S.FIELD_VEL, S.FIELD_DENSITY, S.FIELD_FACTOR, S.FIELD_KAPPA, S.FIELD_ACC)])
+        s.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
