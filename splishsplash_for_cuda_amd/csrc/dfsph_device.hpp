@@ -112,7 +112,9 @@ struct HostRecord {
     DevTime tm;
     uint32_t max_seen, overflow, unstaged_blocks, escaped;
     unsigned long long nbr_fluid, nbr_boundary, nbr_fluid_unstaged;
-    uint32_t seq, pad[3];
+    uint32_t seq;
+    uint32_t count_seq, count;     // a count on its own (k_publish_count), count_seq written last
+    uint32_t pad;
 };
 
 // A Jacobi loop's control, set by the first sweep of its solve (block 0)

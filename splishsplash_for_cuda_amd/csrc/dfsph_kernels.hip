@@ -67,6 +67,16 @@ __device__ void publish(const Publish& pub, const SolveCtl* sc)
     __hip_atomic_store(&r->seq, pub.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// A count the host waits for, published as the loop state is.
+__global__ void k_publish_count(const uint32_t* count, HostRecord* r, uint32_t seq)
+{
+    if (threadIdx.x == 0) {
+        r->count = *count;
+        __threadfence_system();
+        __hip_atomic_store(&r->count_seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // DFSPHCData::reset time bookkeeping (DFSPH_c_arrays_structure.cpp:1000-1004)
 __global__ void k_time_reset(DevTime* t, double h)
 {
@@ -1853,6 +1863,11 @@ void launch_exclusive_scan(hipStream_t s, uint32_t* in, uint32_t* out, uint32_t 
 }
 
 void launch_nbr_ctl_init(hipStream_t s, DevCtl* c) { k_nbr_ctl_init<<<1, 64, 0, s>>>(c); }
+
+void launch_publish_count(hipStream_t s, const uint32_t* count, HostRecord* rec, uint32_t seq)
+{
+    k_publish_count<<<1, 64, 0, s>>>(count, rec, seq);
+}
 
 void launch_time_reset(hipStream_t s, DevTime* t, double h) { k_time_reset<<<1, 64, 0, s>>>(t, h); }
 

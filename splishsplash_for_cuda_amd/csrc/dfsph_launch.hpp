@@ -29,6 +29,7 @@ void launch_exclusive_scan(hipStream_t s, uint32_t* in, uint32_t* out, uint32_t 
                            bool clear_in = false);
 
 void launch_nbr_ctl_init(hipStream_t s, DevCtl* c);
+void launch_publish_count(hipStream_t s, const uint32_t* count, HostRecord* rec, uint32_t seq);
 void launch_time_reset(hipStream_t s, DevTime* t, double h);
 void launch_time_update(hipStream_t s, DevTime* t, double hf, DevCtl* ctl, const float* partial, uint32_t n, int mode,
                         double cfl_factor, double diameter, double dt_min, double dt_max, double seed);
@@ -120,10 +121,10 @@ void launch_outflow_keep(hipStream_t s, const float4* p, uint32_t n, const Surfa
                          uint32_t* keep);
 void launch_inflow(hipStream_t s, const SimConst& c, const float4* cand, uint32_t nc, const float4* pos,
                    const float4* vel, const uint32_t* cs_f, const uint32_t* perm, const float4* bpos,
-                   const uint32_t* cs_b, const Surface& boundary, float min_dist, float max_density, float mass,
+                   const uint32_t* cs_b, const Surface& boundary, float min_dist, float max_density,
                    uint32_t* keep, float4* vel_out);
 void launch_append_inflow(hipStream_t s, const float4* cand, uint32_t nc, const uint32_t* keep, const uint32_t* rank,
-                          const float4* vnew, uint32_t n, float mass, uint32_t first_id, const FluidPtrs& f);
+                          const float4* vnew, uint32_t n, uint32_t first_id, const FluidPtrs& f);
 void launch_apply_delta(hipStream_t s, float4* p, uint32_t n, float dx, float dy, float dz);
 void launch_count_tag(hipStream_t s, const uint32_t* tag, uint32_t n, uint32_t t, uint32_t* count);
 void launch_tag_neighbors(hipStream_t s, const SimConst& c, uint32_t n, const NbrLists& L, const uint32_t* src,

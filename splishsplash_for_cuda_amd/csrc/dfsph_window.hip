@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kInflowBlock) void k_inflow(SimConst c, const float
                                                    const uint32_t* __restrict__ perm,
                                                    const float4* __restrict__ bpos,
                                                    const uint32_t* __restrict__ cs_b, Surface boundary,
-                                                   float min_dist, float max_density, float mass,
+                                                   float min_dist, float max_density,
                                                    uint32_t* __restrict__ keep, float4* __restrict__ vel_out)
 {
     __shared__ uint2 s_range[27][kInflowBlock];
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(kInflowBlock) void k_inflow(SimConst c, const float
     uint32_t ok = 0;
     float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (dmin > min_dist) {
-        float dens = c.W0 * mass, sw = 0.0f, vx = 0.0f, vy = 0.0f, vz = 0.0f;
+        float dens = c.W0 * pos[0].w, sw = 0.0f, vx = 0.0f, vy = 0.0f, vz = 0.0f;
 #pragma unroll 1
         for (int r = 0; r < 27; ++r) {
             const uint2 g = s_range[r][threadIdx.x];
@@ -275,13 +275,13 @@ __global__ __launch_bounds__(kInflowBlock) void k_inflow(SimConst c, const float
 // particles (kappa = kappaV = 0, mass of fluid particle 0, fresh ids).
 __global__ void k_append_inflow(const float4* __restrict__ cand, uint32_t nc, const uint32_t* __restrict__ keep,
                                 const uint32_t* __restrict__ rank, const float4* __restrict__ vnew, uint32_t n,
-                                float mass, uint32_t first_id, FluidPtrs f)
+                                uint32_t first_id, FluidPtrs f)
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= nc || !keep[k]) return;
     const uint32_t o = n + rank[k];
     const float4 p = cand[k];
-    f.pos[o] = make_float4(p.x, p.y, p.z, mass);
+    f.pos[o] = make_float4(p.x, p.y, p.z, f.pos[0].w);
     f.vel[o] = vnew[k];
     f.kap[o] = 0.0f;
     f.kapv[o] = 0.0f;
@@ -482,17 +482,17 @@ void launch_outflow_keep(hipStream_t s, const float4* p, uint32_t n, const Surfa
 
 void launch_inflow(hipStream_t s, const SimConst& c, const float4* cand, uint32_t nc, const float4* pos,
                    const float4* vel, const uint32_t* cs_f, const uint32_t* perm, const float4* bpos,
-                   const uint32_t* cs_b, const Surface& boundary, float min_dist, float max_density, float mass,
+                   const uint32_t* cs_b, const Surface& boundary, float min_dist, float max_density,
                    uint32_t* keep, float4* vel_out)
 {
     k_inflow<<<(nc + kInflowBlock) / kInflowBlock, kInflowBlock, 0, s>>>(c, cand, nc, pos, vel, cs_f, perm, bpos, cs_b, boundary, min_dist,
-                                            max_density, mass, keep, vel_out);
+                                            max_density, keep, vel_out);
 }
 
 void launch_append_inflow(hipStream_t s, const float4* cand, uint32_t nc, const uint32_t* keep, const uint32_t* rank,
-                          const float4* vnew, uint32_t n, float mass, uint32_t first_id, const FluidPtrs& f)
+                          const float4* vnew, uint32_t n, uint32_t first_id, const FluidPtrs& f)
 {
-    if (nc) k_append_inflow<<<nb_(nc), kBlock, 0, s>>>(cand, nc, keep, rank, vnew, n, mass, first_id, f);
+    if (nc) k_append_inflow<<<nb_(nc), kBlock, 0, s>>>(cand, nc, keep, rank, vnew, n, first_id, f);
 }
 
 void launch_apply_delta(hipStream_t s, float4* p, uint32_t n, float dx, float dy, float dz)

@@ -69,3 +69,25 @@ def test_cfl_over_block_maxima(n):
         assert dt == pytest.approx(want, rel=1e-6)
         assert s.cfl(1e-6, 1.0, 1.0) == dt
         s.close()
+
+
+@pytest.mark.parametrize("dropped", [0, 1, 500, "all but one"])
+def test_counts_between_steps(dropped):
+    """Counts the host waits for (removals, loaded fluid) between steps whose state is
+    waited for too; loaded particles take the mass of fluid particle 0."""
+    s = _solver()
+    s.step()
+    n = len(s.download(S.FIELD_ID))
+    keep = np.ones(n, np.uint8)
+    keep[np.random.default_rng(5).permutation(n)[:n - 1 if dropped == "all but one" else dropped]] = 0
+    ids = s.download(S.FIELD_ID)
+    assert s.remove_particles(keep) == keep.sum()
+    assert np.array_equal(s.download(S.FIELD_ID), ids[keep == 1])
+    r = 0.025
+    cand = np.array([[0.75, 1.0, 0.3], [0.8, 1.0, 0.3], [0.85, 1.0, 0.3]], np.float32)   # above the block
+    assert s.load_fluid(np.concatenate([cand, s.download(S.FIELD_POS)[:1]]), 0.5 * r, 1e9) == 3
+    m = s.download(S.FIELD_MASS)
+    assert len(m) == keep.sum() + 3 and np.array_equal(m[-3:], np.repeat(m[0], 3))
+    st = s.step()
+    assert st.n_fluid == len(m) and st.iters >= 2
+    s.close()
