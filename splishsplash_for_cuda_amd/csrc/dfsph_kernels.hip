@@ -432,10 +432,9 @@ struct ListWriter32 {
 // three cells x-1..x+1 of any row are consecutive: one contiguous range of
 // the set per row.
 // LDS of the search with 512-particle blocks: 2688 staged positions (12 B each)
-// and 512 set cells take 40 KB (sets above that search through global
-// memory).  Sparse blocks (spray) have many cells and few particles: tables of
-// up to kBigCells cells take the upper half of the stage when the set fits the
-// lower half.
+// and 512 set cells take 40 KB (larger sets pass through the stage in windows).
+// Sparse blocks (spray) have many cells and few particles: tables of up to
+// kBigCells cells take the upper half of the stage, the lower one holds positions.
 #ifndef DFSPH_NBR_STAGE
 #define DFSPH_NBR_STAGE (DFSPH_BLOCK == 512 ? 2688 : 2048)
 #endif
@@ -521,10 +520,8 @@ __device__ __forceinline__ uint32_t lowest_bits(uint32_t m, uint32_t count)
 }
 
 // visit(q, position of at(q)) for q in [s0, e), four positions loaded at a time:
-// the search of what its stage does not hold is one lane's chain of reads, and
-// the few blocks it happens to outlast the others (one read at a time -> four:
-// 258k particles 97 -> 83 us, with walls at spacing r 184 -> 142, 200k with spray
-// 117 -> 96; eight do not fit 64 registers).
+// the search of blocks without tables or 16-bit lists is one lane's chain of
+// reads, and these few blocks outlast the others (eight do not fit 64 registers).
 constexpr uint32_t kScanBatch = 4;
 template <class At, class Visit>
 __device__ __forceinline__ void scan_positions(const float4* __restrict__ pos, uint32_t s0, uint32_t e, At&& at, Visit&& visit)
@@ -550,10 +547,10 @@ __device__ __forceinline__ void scan_positions(const float4* __restrict__ pos, u
 // Each block also builds its neighbor set: the set cells are marked in the
 // row masks, numbered by a block scan over the rows, and get their fluid
 // ranges, set offsets and boundary ranges, one thread per cell.  Every lane then
-// keeps its 9 rows as (first, last) set cells in registers.  Sets up to
-// kNbrStage have their positions staged in LDS for the candidate tests (over
-// the masks, which are dead by then); sets up to kStageCap store 16-bit lists;
-// larger ones, blocks whose tables do not fit, and the INDIRECT search (fluid
+// keeps its 9 rows as (first, last) set cells in registers.  The set's positions
+// are staged in LDS for the candidate tests (over the masks, which are dead by
+// then), with the boundary's behind them where both fit.  Sets up to kStageCap
+// store 16-bit lists; larger ones, blocks whose tables do not fit, and the INDIRECT search (fluid
 // not reordered, the grid indexes it through perm: the need_sort == false
 // path) store 32-bit global lists.
 //
@@ -767,48 +764,57 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
         }
         __syncthreads();
     }
-    uint32_t total = 0, trunc = 0, stored_f = 0, stored_b = 0, stored_u32 = 0;
-    if (act && mine && !is_source(rs, i)) cnt[i] = 0;   // restricted out: no lists
-    if (act && mine && is_source(rs, i)) {
-        const uint32_t maxn = c.max_nbr, cap = c.cap;
-        const float hk2 = c.hk2;
-        uint32_t nf = 0, nb = 0;                 // found; stored while below max_neighbors
+    const bool searches = act && mine && is_source(rs, i);
+    if (act && mine && !searches) cnt[i] = 0;   // restricted out: no lists
+    const uint32_t maxn = c.max_nbr, cap = c.cap;
+    const float hk2 = c.hk2;
+    uint32_t nf = 0, nb = 0;                     // found; stored while below max_neighbors
+    // Each row range goes in chunks of up to 32 candidates: a branch-free pass
+    // sets one bit per candidate within h, then the set bits are appended in
+    // order.  [s0, e): the range in the stage, which holds the set from w0 on.
+    auto fluid_range = [&](ListWriter16& w, uint32_t self, uint32_t s0, uint32_t e, uint32_t w0) {
+        for (uint32_t l0 = s0 & ~1u; l0 < e; l0 += 32u) {
+            uint32_t m = near_mask(st, p, hk2, l0, e);
+            if (l0 < s0) m &= ~1u;               // the position before the range
+            if (self - w0 - l0 < 32u) m &= ~(1u << (self - w0 - l0));
+            const uint32_t hits = (uint32_t)__popc(m);
+            if (nf + hits > maxn) m = lowest_bits(m, nf < maxn ? maxn - nf : 0u);
+            nf += hits;
+            for (; m != 0u; m &= m - 1u) w.push((w0 + l0 + (uint32_t)__builtin_ctz(m)) << 4);   // LDS byte offset
+        }
+    };
+    if (S != kUnstaged && !lds_search) {
+        // Sets beyond the stage pass through it in windows, each lane's rows cut
+        // to the window; the set's order is the rows' order, so the lists
+        // are the same.  With the walls below, against four global reads at a time:
+        // the wave tank's search (260k) 81 -> 66 us, 258k particles with walls at
+        // spacing r 142 -> 128, 200k with spray 95 -> 85 (4.19 M: 438 -> 442).
+        ListWriter16 w{reinterpret_cast<uint4*>(nbr16) + i, cap};
+        const uint32_t self = searches ? i - s_src[uown] : 0u;
+        for (uint32_t w0 = 0; w0 < S; w0 += room) {
+            const uint32_t w1 = min(w0 + room, S);
+            __syncthreads();                     // the window before is read
+            for (uint32_t u = threadIdx.x >> 3; u < U; u += kBlock / 8) {
+                const uint32_t e = min(s_off[u + 1u], w1), g0 = s_src[u];
+                for (uint32_t k = max(s_off[u], w0) + (threadIdx.x & 7u); k < e; k += 8u) st.put(k - w0, pos[g0 + k]);
+            }
+            __syncthreads();
+#pragma unroll 1
+            for (int r = 0; r < 9; ++r) {
+                if (!searches || row[r] == kNoRow) continue;
+                const uint32_t s0 = max(s_off[row[r] & 0xffffu], w0), e = min(s_off[(row[r] >> 16) + 1u], w1);
+                if (s0 < e) fluid_range(w, self, s0 - w0, e - w0, w0);
+            }
+        }
+        if (searches) w.finish();
+    } else if (searches) {
         if (S != kUnstaged) {
             ListWriter16 w{reinterpret_cast<uint4*>(nbr16) + i, cap};
             const uint32_t self = i - s_src[uown];
-            if (lds_search) {
-                // Each row range goes in chunks of up to 32 candidates: a branch-free
-                // pass sets one bit per candidate within h, then the set bits
-                // are appended in order.
 #pragma unroll 1
-                for (int r = 0; r < 9; ++r) {
-                    if (row[r] == kNoRow) continue;
-                    const uint32_t s0 = s_off[row[r] & 0xffffu], e = s_off[(row[r] >> 16) + 1u];
-                    for (uint32_t l0 = s0 & ~1u; l0 < e; l0 += 32u) {
-                        uint32_t m = near_mask(st, p, hk2, l0, e);
-                        if (l0 < s0) m &= ~1u;           // the position before the range
-                        if (self - l0 < 32u) m &= ~(1u << (self - l0));
-                        const uint32_t hits = (uint32_t)__popc(m);
-                        if (nf + hits > maxn) m = lowest_bits(m, nf < maxn ? maxn - nf : 0u);
-                        nf += hits;
-                        for (; m != 0u; m &= m - 1u) w.push((l0 + (uint32_t)__builtin_ctz(m)) << 4);   // LDS byte offset
-                    }
-                }
-            } else {
-#pragma unroll 1
-                for (int r = 0; r < 9; ++r) {
-                    if (row[r] == kNoRow) continue;
-                    for (uint32_t u = row[r] & 0xffffu; u <= (row[r] >> 16); ++u) {
-                        const uint32_t src = s_src[u];
-                        scan_positions(pos, s_off[u], s_off[u + 1u], [&](uint32_t l) { return src + l; },
-                                       [&](uint32_t l, const float4& qp) {
-                            if (dist2(p.x - qp.x, p.y - qp.y, p.z - qp.z) < hk2 && l != self) {
-                                if (nf < maxn) w.push(l << 4);
-                                ++nf;
-                            }
-                        });
-                    }
-                }
+            for (int r = 0; r < 9; ++r) {
+                if (row[r] == kNoRow) continue;
+                fluid_range(w, self, s_off[row[r] & 0xffffu], s_off[(row[r] >> 16) + 1u], 0u);
             }
             w.finish();
         } else {
@@ -837,51 +843,63 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
             }
             w.finish();
         }
-        const uint32_t sf = nf < maxn ? nf : maxn;
-        ListWriter32 wb{reinterpret_cast<uint4*>(nbrb) + i, cap};
-        auto scan_boundary = [&](uint32_t s0, uint32_t e) {
+    }
+    const uint32_t sf = nf < maxn ? nf : maxn;
+    ListWriter32 wb{reinterpret_cast<uint4*>(nbrb) + i, cap};
+    // A row's boundary particles are one contiguous staged range, in up to
+    // three runs of boundary indices (one per cell).  at: what the stage begins
+    // with; [w0, w1): the boundary offsets that follow it.
+    auto boundary_row = [&](uint32_t rw, uint32_t at, uint32_t w0, uint32_t w1) {
+        const uint32_t u0 = rw & 0xffffu, u1 = rw >> 16;
+        const uint32_t b0 = max(s_boff[u0], w0), b1 = min(s_boff[u1 + 1u], w1);
+        if (b0 >= b1) return;
+        const uint32_t mv = at - w0, s0 = b0 + mv, e = b1 + mv;
+        const uint32_t ub = min(u0 + 1u, u1), k1 = s_boff[ub] + mv, k2 = s_boff[u1] + mv;
+        const uint32_t j0 = s_bs[u0] - mv, j1 = s_bs[ub] - mv, j2 = s_bs[u1] - mv;
+        for (uint32_t l0 = s0 & ~1u; l0 < e; l0 += 32u) {
+            uint32_t m = near_mask(st, p, hk2, l0, e);
+            if (l0 < s0) m &= ~1u;               // the position before the range
+            const uint32_t hits = (uint32_t)__popc(m);
+            if (sf + nb + hits > maxn) m = lowest_bits(m, sf + nb < maxn ? maxn - sf - nb : 0u);
+            nb += hits;
+            for (; m != 0u; m &= m - 1u) {
+                const uint32_t k = l0 + (uint32_t)__builtin_ctz(m);
+                wb.push(k + ((int)(k - k1) < 0 ? j0 : (int)(k - k2) < 0 ? j1 : j2));
+            }
+        }
+    };
+    if (lds_bnd) {
+        if (Sb > 0u && searches) {
+#pragma unroll 1
+            for (int r = 0; r < 9; ++r)
+                if (row[r] != kNoRow) boundary_row(row[r], S, 0u, Sb);
+        }
+    } else if (tabled) {
+        // the walls after the fluid, in windows of the stage
+        for (uint32_t w0 = 0; w0 < Sb; w0 += room) {
+            const uint32_t w1 = min(w0 + room, Sb);
+            __syncthreads();                     // the stage's last contents are read
+            for (uint32_t u = threadIdx.x >> 3; u < U; u += kBlock / 8) {
+                const uint32_t e = min(s_boff[u + 1u], w1), j0 = s_bs[u];
+                for (uint32_t k = max(s_boff[u], w0) + (threadIdx.x & 7u); k < e; k += 8u) st.put(k - w0, bpos[j0 + k]);
+            }
+            __syncthreads();
+#pragma unroll 1
+            for (int r = 0; r < 9; ++r)
+                if (searches && row[r] != kNoRow) boundary_row(row[r], 0u, w0, w1);
+        }
+    } else if (searches) {
+        for_each_adjacent_range(c, cx, cy, cz, cs_b, [&](uint32_t s0, uint32_t e) {
             scan_positions(bpos, s0, e, [](uint32_t j) { return j; }, [&](uint32_t j, const float4& pj) {
                 if (dist2(p.x - pj.x, p.y - pj.y, p.z - pj.z) < hk2) {
                     if (sf + nb < maxn) wb.push(j);
                     ++nb;
                 }
             });
-        };
-        if (lds_bnd) {
-            // the row's boundary particles are one contiguous staged range, in
-            // up to three runs of boundary indices (one per cell)
-            if (Sb > 0u) {
-#pragma unroll 1
-                for (int r = 0; r < 9; ++r) {
-                    if (row[r] == kNoRow) continue;
-                    const uint32_t u0 = row[r] & 0xffffu, u1 = row[r] >> 16;
-                    const uint32_t s0 = S + s_boff[u0], e = S + s_boff[u1 + 1u];
-                    if (s0 == e) continue;
-                    const uint32_t ub = min(u0 + 1u, u1), k1 = S + s_boff[ub], k2 = S + s_boff[u1];
-                    const uint32_t j0 = s_bs[u0] - S, j1 = s_bs[ub] - S, j2 = s_bs[u1] - S;
-                    for (uint32_t l0 = s0 & ~1u; l0 < e; l0 += 32u) {
-                        uint32_t m = near_mask(st, p, hk2, l0, e);
-                        if (l0 < s0) m &= ~1u;           // the position before the range
-                        const uint32_t hits = (uint32_t)__popc(m);
-                        if (sf + nb + hits > maxn) m = lowest_bits(m, sf + nb < maxn ? maxn - sf - nb : 0u);
-                        nb += hits;
-                        for (; m != 0u; m &= m - 1u) {
-                            const uint32_t k = l0 + (uint32_t)__builtin_ctz(m);
-                            wb.push(k + (k < k1 ? j0 : k < k2 ? j1 : j2));
-                        }
-                    }
-                }
-            }
-        } else if (tabled) {
-#pragma unroll 1
-            for (int r = 0; r < 9; ++r) {
-                if (row[r] == kNoRow) continue;
-                for (uint32_t u = row[r] & 0xffffu; u <= (row[r] >> 16); ++u)
-                    scan_boundary(s_bs[u] + s_boff[u], s_bs[u] + s_boff[u + 1u]);
-            }
-        } else {
-            for_each_adjacent_range(c, cx, cy, cz, cs_b, scan_boundary);
-        }
+        });
+    }
+    uint32_t total = 0, trunc = 0, stored_f = 0, stored_b = 0, stored_u32 = 0;
+    if (searches) {
         const uint32_t sb = nb < maxn - sf ? nb : maxn - sf;
         wb.finish();
         total = nf + nb;

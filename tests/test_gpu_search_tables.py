@@ -183,3 +183,26 @@ def test_streamed_lists(n):
         s.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("fluid, wall", [(1.2, 2.0), (1.2, 0.7), (2.0, 0.6)])
+def test_search_windows(fluid, wall):
+    """Sets and walls that pass through the stage in windows (spacings in radii: two
+    windows of the set, then of the walls too, then of the walls alone): each list's members by a k-d
+    tree, in the order of the cells, with and without LDS-staged sweeps."""
+    from scipy.spatial import cKDTree
+    rng = np.random.default_rng(int(100 * fluid + wall))
+    x = _jitter(fluid_block((0.05, 0.05, 0.05), (13, 14, 15), fluid * R), rng, 0.2).astype(np.float32)
+    walls = box_surface((0, 0, 0), (0.8, 0.8, 0.8), wall * R).astype(np.float32)
+    pos, bpos, nf, nb, L, stats = _search(x, walls, 255, S.LISTS_AUTO)
+    for mode in (S.LISTS_NO_LDS, S.LISTS_GLOBAL):
+        other = _search(x, walls, 255, mode)
+        assert np.array_equal(nf, other[2]) and np.array_equal(nb, other[3]) and np.array_equal(L, other[4])
+    p, q = pos.astype(np.float64), bpos.astype(np.float64)
+    lo_f, hi_f = (cKDTree(p).query_ball_point(p, H * (1 + e)) for e in (-1e-5, 1e-5))
+    lo_b, hi_b = (cKDTree(q).query_ball_point(p, H * (1 + e)) for e in (-1e-5, 1e-5))
+    assert (nf + nb).max() < 255                # no list is truncated
+    for i in range(len(p)):
+        f, b = L[i, :nf[i]], L[i, nf[i]:nf[i] + nb[i]]
+        assert set(lo_f[i]) - {i} <= set(f) <= set(hi_f[i]) - {i} and len(set(f)) == len(f)
+        assert set(lo_b[i]) <= set(b) <= set(hi_b[i]) and len(set(b)) == len(b)
