@@ -441,7 +441,11 @@ struct ListWriter32 {
 constexpr uint32_t kNbrStage = DFSPH_NBR_STAGE;   // set positions staged in LDS by the search
 static_assert(kNbrStage % 16 == 0, "halves, and rows in whole words");
 constexpr uint32_t kHalfStage = kNbrStage / 2;
-constexpr uint32_t kSetRows = kHalfStage * 3 / 4; // rows (y, z) of a tabled set's bounding box
+// Rows (y, z) of a tabled set's bounding box.  34 x 34 of them hold the set of a
+// block that runs from one octant of a 32-cell cube to the next (1008 did not:
+// the few such blocks searched cell by cell, and of 258k particles the whole
+// search waited for them, 82 us against 54).
+constexpr uint32_t kSetRows = kHalfStage * 9 / 10 & ~1u;
 #ifndef DFSPH_SET_CELLS
 #define DFSPH_SET_CELLS (DFSPH_BLOCK == 512 ? 512 : 384)
 #endif
@@ -577,12 +581,14 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
     __shared__ __align__(16) PosStage st;
     unsigned long long* s_mask = reinterpret_cast<unsigned long long*>(st.d);   // x positions of the row's set cells
     uint32_t* s_place = reinterpret_cast<uint32_t*>(s_mask + kSetRows);   // box place of a set cell: x | z << 6 | y << 16
-    uint16_t* s_first = reinterpret_cast<uint16_t*>(s_place + kBigCells); // number of the row's first set cell
-    static_assert(kSetRows * 10 + kBigCells * 4 <= kHalfStage * 12, "tables under construction exceed half the stage");
+    uint16_t* s_first = reinterpret_cast<uint16_t*>(s_place + kSetCells); // number of the row's first set cell
+    static_assert(kSetRows * 10 + kSetCells * 4 <= kHalfStage * 12 && kSetRows * 8 + kBigCells * 4 <= kHalfStage * 12,
+                  "tables under construction exceed half the stage");
     // four words per set cell (one more for the offsets): set offset of its fluid
     // particles and what to add for their indices, the same for its boundary ones
     __shared__ uint32_t s_tab[4 * kSetCells + 2];
-    static_assert(4 * kSetCells + 2 > kBigCells, "the boundary offsets of a large table lie in s_tab");
+    static_assert(4 * kSetCells + 2 >= kBigCells + 1 + kSetRows / 2,
+                  "the boundary offsets of a large table and its rows' first cells lie in s_tab");
     uint32_t *s_off = s_tab, *s_src = s_tab + kSetCells + 1, *s_boff = s_src + kSetCells, *s_bs = s_boff + kSetCells + 1;
     constexpr int NW = kBlock / 64;
     __shared__ int s_w[6 * NW];
@@ -618,7 +624,8 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
             s_w[w] = lo_x; s_w[NW + w] = lo_y; s_w[2 * NW + w] = lo_z;
             s_w[3 * NW + w] = hi_x; s_w[4 * NW + w] = hi_y; s_w[5 * NW + w] = hi_z;
         }
-        for (uint32_t k = threadIdx.x; k < kSetRows; k += kBlock) s_mask[k] = 0ull;
+        for (uint32_t k = threadIdx.x; k < kSetRows / 2; k += kBlock)
+            reinterpret_cast<uint4*>(s_mask)[k] = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
         int lo[3] = {kIntMax, kIntMax, kIntMax}, hi[3] = {-1, -1, -1};
 #pragma unroll
@@ -668,6 +675,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
                 s_src = s_off + kHalfStage;
                 s_bs = s_src + kHalfStage;
                 s_boff = s_tab;
+                s_first = reinterpret_cast<uint16_t*>(s_tab + kBigCells + 1);
             }
             if (tabled) {
                 for (uint32_t k = k0; k < k1; ++k) {

@@ -206,3 +206,22 @@ def test_search_windows(fluid, wall):
         f, b = L[i, :nf[i]], L[i, nf[i]:nf[i] + nb[i]]
         assert set(lo_f[i]) - {i} <= set(f) <= set(hi_f[i]) - {i} and len(set(f)) == len(f)
         assert set(lo_b[i]) <= set(b) <= set(hi_b[i]) and len(set(b)) == len(b)
+
+
+@pytest.mark.parametrize("at", [0.05, 0.2])
+def test_search_across_octants(at):
+    """Blocks that run from one octant of a 32-cell cube to the next, whose set's box has
+    34 x 34 rows: neighbors as a k-d tree counts them, few particles around."""
+    from scipy.spatial import cKDTree
+    rng = np.random.default_rng(int(100 * at))
+    edge = 16 * 1.001 * H                         # between the cube's octants
+    corner = np.stack(np.meshgrid(*[[0.0, edge - 6 * R, edge + 4 * R, 2 * edge - 6 * R]] * 3, indexing="ij"), -1).reshape(-1, 3)
+    x = np.concatenate([_jitter(fluid_block(c, (3, 3, 3), 2 * R), rng, 0.2) for c in corner + at]).astype(np.float32)
+    walls = box_surface((0, 0, 0), (4.0, 4.0, 4.0), 2 * R).astype(np.float32)
+    pos, bpos, nf, nb, L, stats = _search(x, walls, 96, S.LISTS_AUTO)
+    trees = cKDTree(pos.astype(np.float64)), cKDTree(bpos.astype(np.float64))
+    p = pos.astype(np.float64)
+    for r, low in ((H * (1 - 1e-5), True), (H * (1 + 1e-5), False)):
+        wf = trees[0].query_ball_point(p, r, return_length=True) - 1
+        wb = trees[1].query_ball_point(p, r, return_length=True)
+        assert ((wf <= nf) & (wb <= nb)).all() if low else ((wf >= nf) & (wb >= nb)).all()
