@@ -642,12 +642,13 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
             hi[a] = min(__builtin_amdgcn_readfirstlane(hi[a]) + 1, c.dim[a] - 1);
         }
         const uint32_t W = (uint32_t)(hi[0] - lo[0] + 1), D = (uint32_t)(hi[2] - lo[2] + 1), H = (uint32_t)(hi[1] - lo[1] + 1);
-        if (W <= 64u && D <= kSetRows && H <= kSetRows && D * H <= kSetRows) {
-            const uint32_t R = D * H;
-            const int xl = max(cx - 1, 0), xh = min(cx + 1, c.dim[0] - 1);
-            const uint32_t bx = (uint32_t)(xl - lo[0]);                            // first x of my rows, in the box
-            const uint32_t nx = (uint32_t)(xh - xl);
-            const uint32_t own = (uint32_t)(cz - lo[2]) + D * (uint32_t)(cy - lo[1]);
+        const bool fits = W <= 64u && D <= kSetRows && H <= kSetRows && D * H <= kSetRows;
+        const uint32_t R = D * H;
+        const int xl = max(cx - 1, 0), xh = min(cx + 1, c.dim[0] - 1);
+        const uint32_t bx = (uint32_t)(xl - lo[0]);                                // first x of my rows, in the box
+        const uint32_t nx = (uint32_t)(xh - xl);
+        const uint32_t own = (uint32_t)(cz - lo[2]) + D * (uint32_t)(cy - lo[1]);
+        if (fits) {
             // mark the 27 cells, one lane per run of a cell in a wave
             const uint32_t lin = act ? (uint32_t)(cx - lo[0]) + W * own : kKeyInvalid;
             const uint32_t prev = (uint32_t)__builtin_amdgcn_update_dpp((int)kKeyInvalid, (int)lin, 0x138, 0xf, 0xf, false);
@@ -660,7 +661,11 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
                         atomicOr(&s_mask[own + (uint32_t)(r % 3 - 1) + D * (uint32_t)(r / 3 - 1)], bits);
                 }
             }
-            __syncthreads();                    // also: s_w is reused by the scans
+        }
+        // The masks are complete and the boxes in s_w are read: its words are
+        // used again by the scans, or, of a block that does not fit, by the statistics.
+        __syncthreads();
+        if (fits) {
             // number the marked cells row by row; thread t owns rows [tE, tE + E)
             const uint32_t E = (R + kBlock - 1) / kBlock;
             const uint32_t k0 = threadIdx.x * E, k1 = min(k0 + E, R);
