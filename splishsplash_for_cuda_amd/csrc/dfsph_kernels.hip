@@ -471,11 +471,27 @@ __device__ __forceinline__ uint32_t wave_total_u(uint32_t v)
     return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan_u(v), 63);
 }
 
-// m = 2 m + (d2 < limit): the compare's carry joins the shift, two vector
-// instructions per candidate (false for a NaN distance).
-__device__ __forceinline__ uint32_t shift_in_less(uint32_t m, float d2, float limit)
+// m = 2 m + (d < limit) for four distances in turn: the compares' carries join the
+// shifts, two vector instructions per candidate (false for a NaN distance).
+// A vector instruction has to wait two others before it reads a scalar
+// register that one has written, so the compares come first, into registers of
+// their own: three instructions lie between each and the sum that reads it.
+// (Written as m + m + (d < limit) a candidate takes three: a search of 4.19 M
+// particles 486 us, with this 475.)
+__device__ __forceinline__ uint32_t shift_in_less(uint32_t m, float d0, float d1, float d2, float d3, float limit)
 {
-    asm("v_cmp_gt_f32_e32 vcc, %2, %1\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(d2), "s"(limit) : "vcc");
+    unsigned long long c0, c1, c2;
+    asm("v_cmp_gt_f32_e64 %1, %8, %4\n\t"
+        "v_cmp_gt_f32_e64 %2, %8, %5\n\t"
+        "v_cmp_gt_f32_e64 %3, %8, %6\n\t"
+        "v_cmp_gt_f32_e32 vcc, %8, %7\n\t"
+        "v_addc_co_u32_e64 %0, %1, %0, %0, %1\n\t"
+        "v_addc_co_u32_e64 %0, %2, %0, %0, %2\n\t"
+        "v_addc_co_u32_e64 %0, %3, %0, %0, %3\n\t"
+        "v_addc_co_u32_e32 %0, vcc, %0, %0, vcc"
+        : "+v"(m), "=&s"(c0), "=&s"(c1), "=&s"(c2)
+        : "v"(d0), "v"(d1), "v"(d2), "v"(d3), "s"(limit)
+        : "vcc");
     return m;
 }
 
@@ -504,10 +520,8 @@ __device__ __forceinline__ uint32_t near_mask(const PosStage& st, const float4& 
     do {
         const f4 a = *reinterpret_cast<const f4*>(st.d + t), b = *reinterpret_cast<const f4*>(st.d + t + 4),
                  c = *reinterpret_cast<const f4*>(st.d + t + 8);
-        m = shift_in_less(m, dist2(p.x - a[0], p.y - a[2], p.z - b[0]), hk2);
-        m = shift_in_less(m, dist2(p.x - a[1], p.y - a[3], p.z - b[1]), hk2);
-        m = shift_in_less(m, dist2(p.x - b[2], p.y - c[0], p.z - c[2]), hk2);
-        m = shift_in_less(m, dist2(p.x - b[3], p.y - c[1], p.z - c[3]), hk2);
+        m = shift_in_less(m, dist2(p.x - a[0], p.y - a[2], p.z - b[0]), dist2(p.x - a[1], p.y - a[3], p.z - b[1]),
+                          dist2(p.x - b[2], p.y - c[0], p.z - c[2]), dist2(p.x - b[3], p.y - c[1], p.z - c[3]), hk2);
         t += 12u;
     } while (t < end);
     // (cnt + 3) / 4 steps made, the first candidate in the highest of their bits

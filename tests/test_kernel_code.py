@@ -84,3 +84,44 @@ def test_search_barrier_between_boxes_and_statistics(kernels):
     last = {body[k][0] for k in barriers if None in _barriers_after(body, k)}
     assert last and body[barriers[0]][0] not in last
     assert not _barriers_after(body, barriers[0]) & last
+
+
+def _scalars(operand):
+    """the scalar registers that an operand names"""
+    if re.search(r"\bvcc\b", operand):
+        return {"vcc"}
+    m = re.match(r"-?\|?s\[(\d+):(\d+)\]", operand)
+    if m:
+        return {"s%d" % k for k in range(int(m[1]), int(m[2]) + 1)}
+    m = re.match(r"-?\|?(s\d+)\b", operand)
+    return {m[1]} if m else set()
+
+
+def test_wait_states_behind_scalar_results(kernels):
+    """A vector instruction that reads a scalar register or VCC which another vector instruction has
+    written comes at least three instructions behind it (two wait states, the rule on
+    gfx940 and later): the compiler sees to it, except inside inline assembly."""
+    early, pairs = [], 0
+    for name, body in kernels.items():
+        written = {}                                    # register -> wait states passed since
+        for addr, text, _ in body:
+            op, _, rest = text.partition(" ")
+            operands = [o.strip() for o in rest.split(",")]
+            if op.startswith("v_"):
+                second = re.match(r"v_(add|sub|subrev|addc|subb|subbrev)_co_|v_div_scale|v_mad_[ui]64", op)
+                results = operands[:2] if second else operands[:1]
+                reads = set().union(*map(_scalars, operands[len(results):])) | ({"vcc"} if "div_fmas" in op else set())
+                for r in reads & written.keys():
+                    pairs += 1
+                    if written[r] < 2:
+                        early.append("%s %x: %s" % (name, addr, text))
+            waits = 1 + int(operands[0]) if op == "s_nop" else 1
+            written = {r: w + waits for r, w in written.items() if w < 8}
+            if op.startswith("v_"):
+                written.update((r, 0) for r in set().union(*map(_scalars, results)))
+            else:                                       # a scalar result takes its place
+                for r in _scalars(operands[0]):
+                    written.pop(r, None)
+            if op == "s_branch":
+                written = {}
+    assert pairs > 100 and not early, early[:8]
