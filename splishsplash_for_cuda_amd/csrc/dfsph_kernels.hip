@@ -451,6 +451,12 @@ constexpr uint32_t kSetRows = kHalfStage * 9 / 10 & ~1u;
 #endif
 constexpr uint32_t kSetCells = DFSPH_SET_CELLS;   // set cells with a full stage
 constexpr uint32_t kBigCells = kHalfStage - 1;    // set cells with half a stage
+// Box place of a set cell in a word, x | z << 6 | y << 16, and the widest box whose
+// places it holds (kSetRows bounds z too, but only in boxes of two rows in y and more).
+constexpr uint32_t kPlaceZ = 6, kPlaceY = 16;
+constexpr uint32_t kBoxW = 1u << kPlaceZ, kBoxD = 1u << (kPlaceY - kPlaceZ);
+static_assert(kBoxW == 64, "a row's mask has 64 bits");
+static_assert(kSetRows <= 1u << (32 - kPlaceY), "y of a box place");
 constexpr uint32_t kNoRow = 0xffffffffu;
 constexpr int kIntMax = 0x7fffffff;
 
@@ -594,7 +600,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
     // positions and are dead once those are loaded.
     __shared__ __align__(16) PosStage st;
     unsigned long long* s_mask = reinterpret_cast<unsigned long long*>(st.d);   // x positions of the row's set cells
-    uint32_t* s_place = reinterpret_cast<uint32_t*>(s_mask + kSetRows);   // box place of a set cell: x | z << 6 | y << 16
+    uint32_t* s_place = reinterpret_cast<uint32_t*>(s_mask + kSetRows);   // box places of the set cells
     uint16_t* s_first = reinterpret_cast<uint16_t*>(s_place + kSetCells); // number of the row's first set cell
     static_assert(kSetRows * 10 + kSetCells * 4 <= kHalfStage * 12 && kSetRows * 8 + kBigCells * 4 <= kHalfStage * 12,
                   "tables under construction exceed half the stage");
@@ -656,7 +662,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
             hi[a] = min(__builtin_amdgcn_readfirstlane(hi[a]) + 1, c.dim[a] - 1);
         }
         const uint32_t W = (uint32_t)(hi[0] - lo[0] + 1), D = (uint32_t)(hi[2] - lo[2] + 1), H = (uint32_t)(hi[1] - lo[1] + 1);
-        const bool fits = W <= 64u && D <= kSetRows && H <= kSetRows && D * H <= kSetRows;
+        const bool fits = W <= kBoxW && D <= kBoxD && H <= kSetRows && D * H <= kSetRows;
         const uint32_t R = D * H;
         const int xl = max(cx - 1, 0), xh = min(cx + 1, c.dim[0] - 1);
         const uint32_t bx = (uint32_t)(xl - lo[0]);                                // first x of my rows, in the box
@@ -698,7 +704,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
             }
             if (tabled) {
                 for (uint32_t k = k0; k < k1; ++k) {
-                    const uint32_t y = k / D, at = ((k - y * D) << 6) | (y << 16);
+                    const uint32_t y = k / D, at = ((k - y * D) << kPlaceZ) | (y << kPlaceY);
                     s_first[k] = (uint16_t)ubase;
                     for (unsigned long long m = s_mask[k]; m != 0ull; m &= m - 1ull)
                         s_place[ubase++] = at | (uint32_t)(__ffsll((long long)m) - 1);
@@ -714,8 +720,8 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
                     cf[k] = cb[k] = f0s[k] = b0s[k] = 0u;
                     if (k < C && u < U) {
                         const uint32_t at = s_place[u];
-                        const uint32_t key = cell_key(c, lo[0] + (int)(at & 63u), lo[1] + (int)(at >> 16),
-                                                      lo[2] + (int)((at >> 6) & 1023u));
+                        const uint32_t key = cell_key(c, lo[0] + (int)(at & (kBoxW - 1u)), lo[1] + (int)(at >> kPlaceY),
+                                                      lo[2] + (int)((at >> kPlaceZ) & (kBoxD - 1u)));
                         const uint32_t f0 = cs_f[key], f1 = cs_f[key + 1], b0 = cs_b[key], b1 = cs_b[key + 1];
                         f0s[k] = f0;
                         b0s[k] = b0;
