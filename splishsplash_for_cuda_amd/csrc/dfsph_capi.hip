@@ -145,6 +145,7 @@ struct Handle {
     bool pend_vel = false;            // deferred cuda_update_vel (fused into the pressure warm start)
     bool lists_valid = false;
     int lists_rmode = 0;              // restriction mode the lists were built under
+    bool lists_sets = false;          // blocks of the lists may have neighbor sets
     bool acc_valid = false;
     bool pred_valid = false;          // features / predictions of this step computed
     // learned warm start gate: the warm-start mode of the current step (set by
@@ -343,7 +344,7 @@ dfsph::NbrLists lists(const Handle* h)
 {
     const dfsph::Solids sol{h->ns ? h->bvel : nullptr, h->sforce, h->fscale};
     return dfsph::NbrLists{h->nbr16, h->nbrf, h->nbrb, h->cnt, h->stage_n, h->stg, restriction(h), sol,
-                           dfsph::list_stream(h->n)};
+                           dfsph::list_stream(h->n), h->lists_sets ? 1u : 0u};
 }
 
 int ensure_scan(Handle* h, uint32_t n)
@@ -472,6 +473,7 @@ int neighbor_search(Handle* h, bool sort)
     HIPCHK(hipGetLastError());
     h->lists_valid = true;
     h->lists_rmode = h->rmode;
+    h->lists_sets = sort && h->c.stage_cap > 0u;
     h->acc_valid = false;
     h->nbr_op = h->ops;
     h->ws_step_set = false;

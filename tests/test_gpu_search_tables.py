@@ -225,3 +225,29 @@ def test_search_across_octants(at):
         wf = trees[0].query_ball_point(p, r, return_length=True) - 1
         wb = trees[1].query_ball_point(p, r, return_length=True)
         assert ((wf <= nf) & (wb <= nb)).all() if low else ((wf >= nf) & (wb >= nb)).all()
+
+
+@pytest.mark.parametrize("name", ["n=513", "spray", "dense walls"])
+def test_sweeps_between_sorted_and_unsorted_searches(name):
+    """Solves on the lists of an unsorted search (no block has a set) between solves on
+    sorted ones: the same bits as with 32-bit lists throughout."""
+    x, walls, maxn = _scene(name, np.random.default_rng(14))
+    v = np.random.default_rng(15).normal(scale=0.3, size=x.shape).astype(np.float32)
+    out = []
+    for mode in (S.LISTS_AUTO, S.LISTS_GLOBAL):
+        s = S.Solver(S.default_params(particle_radius=R, max_neighbors=maxn, list_mode=mode))
+        s.upload_boundary(walls)
+        s.upload_fluid(x, v)
+        fields = []
+        for sort in (True, False, False, True):
+            s.neighbor_search(sort)
+            s.divergence_solve(3, 0.0)
+            s.external_forces()
+            s.update_vel()
+            s.pressure_solve(2, 0.0)
+            fields += [s.download(f) for f in (S.FIELD_ID, S.FIELD_VEL, S.FIELD_DENSITY, S.FIELD_FACTOR, S.FIELD_KAPPA,
+                                               S.FIELD_KAPPAV, S.FIELD_ACC)]
+        out.append(fields)
+        s.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b, equal_nan=True)
