@@ -543,21 +543,30 @@ __device__ __forceinline__ uint32_t lowest_bits(uint32_t m, uint32_t count)
     return r;
 }
 
-// visit(q, position of at(q)) for q in [s0, e), four positions loaded at a time:
-// the search of blocks without tables or 16-bit lists is one lane's chain of
-// reads, and these few blocks outlast the others (eight do not fit 64 registers).
+// visit(q, position of at(q)) for q in [s0, e), four positions loaded at a time (eight do
+// not fit 64 registers): the search of blocks without tables or 16-bit
+// lists is one lane's chain of reads.  REST: what is left of a range singly.  Cells hold
+// 8 to 12 particles, and a masked batch wastes up to three tests of each, which the
+// few blocks that outlast a sorted search do not feel (the sparsest spray 69 us, with the rest singly 70),
+// but an unsorted search does, where every block reads so: 150k particles
+// 177 us masked, 139 with the rest singly, 1.05 M 552 and 463.
 constexpr uint32_t kScanBatch = 4;
-template <class At, class Visit>
+template <bool REST, class At, class Visit>
 __device__ __forceinline__ void scan_positions(const float4* __restrict__ pos, uint32_t s0, uint32_t e, At&& at, Visit&& visit)
 {
+    uint32_t q = s0;
 #pragma unroll 1
-    for (uint32_t q = s0; q < e; q += kScanBatch) {
+    for (; REST ? q + kScanBatch <= e : q < e; q += kScanBatch) {
         float4 t[kScanBatch];
 #pragma unroll
-        for (uint32_t u = 0; u < kScanBatch; ++u) t[u] = pos[at(min(q + u, e - 1u))];
+        for (uint32_t u = 0; u < kScanBatch; ++u) t[u] = pos[at(REST ? q + u : min(q + u, e - 1u))];
 #pragma unroll
         for (uint32_t u = 0; u < kScanBatch; ++u)
-            if (q + u < e) visit(q + u, t[u]);
+            if (REST || q + u < e) visit(q + u, t[u]);
+    }
+    if (REST) {
+#pragma unroll 1
+        for (; q < e; ++q) visit(q, pos[at(q)]);
     }
 }
 
@@ -854,7 +863,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
             ListWriter32 w{reinterpret_cast<uint4*>(nbrf) + i, cap};
             auto scan_range = [&](uint32_t s0, uint32_t e) {
                 auto index = [&](uint32_t q) { return INDIRECT ? perm[q] : q; };
-                scan_positions(pos, s0, e, index, [&](uint32_t q, const float4& pj) {
+                scan_positions<INDIRECT>(pos, s0, e, index, [&](uint32_t q, const float4& pj) {
                     if (dist2(p.x - pj.x, p.y - pj.y, p.z - pj.z) < hk2) {
                         const uint32_t j = index(q);
                         if (j != i) {
@@ -923,7 +932,7 @@ __global__ __launch_bounds__(kBlock, DFSPH_BLOCK == 512 ? 8 : 4) void k_neighbor
         }
     } else if (searches) {
         for_each_adjacent_range(c, cx, cy, cz, cs_b, [&](uint32_t s0, uint32_t e) {
-            scan_positions(bpos, s0, e, [](uint32_t j) { return j; }, [&](uint32_t j, const float4& pj) {
+            scan_positions<INDIRECT>(bpos, s0, e, [](uint32_t j) { return j; }, [&](uint32_t j, const float4& pj) {
                 if (dist2(p.x - pj.x, p.y - pj.y, p.z - pj.z) < hk2) {
                     if (sf + nb < maxn) wb.push(j);
                     ++nb;

@@ -251,3 +251,26 @@ def test_sweeps_between_sorted_and_unsorted_searches(name):
         s.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("name", ["n=1", "n=2", "n=513", "spray", "rows over 32", "dense walls", "truncated"])
+def test_unsorted_search(name):
+    """The search of fluid left in its order, here a shuffled one, cells of every size: the
+    lists of the sorted search, as ids and in the same order."""
+    x, walls, maxn = _scene(name, np.random.default_rng(16))
+    x = x[np.random.default_rng(17).permutation(len(x))]
+    s = S.Solver(S.default_params(particle_radius=R, max_neighbors=maxn))
+    s.upload_boundary(walls)
+    s.upload_fluid(x)
+    s.neighbor_search(False)
+    assert np.array_equal(s.download(S.FIELD_POS), x)
+    nf, nb, L = s.neighbors()
+    s.neighbor_search()
+    ids = s.download(S.FIELD_ID)
+    sf, sb, G = s.neighbors()
+    s.close()
+    assert np.array_equal(nf[ids], sf) and np.array_equal(nb[ids], sb) and sf.max() >= (len(x) > 2)
+    for k, i in enumerate(ids):
+        f = int(sf[k])
+        assert np.array_equal(ids[G[k, :f]], L[i, :f])
+        assert np.array_equal(G[k, f:f + int(sb[k])], L[i, f:f + int(sb[k])])
