@@ -497,9 +497,6 @@ int step_warm_start(Handle* h)
     return h->ws_step;
 }
 
-// Queue Jacobi iterations in batches; the device decides when the loop ends
-// (kernels of later iterations exit at once).  Two readback slots keep one
-// batch in flight while the previous batch's loop state is inspected.
 // The loop control a solve's first sweep sets (block 0 of that sweep).
 dfsph::CtlInit solve_ctl(Handle* h, bool div, uint32_t max_iter, double max_error)
 {
@@ -576,7 +573,7 @@ int jacobi_loop(Handle* h, bool div, uint32_t max_iter, double max_error, uint32
         HIPCHK(hipGetLastError());
         CHK(wait_record(h, h->seq));
         res = h->last.sc;
-        if (res.done) pdrop(h, pr);   // that sweep exited at once
+        if (res.done) pdrop(h, pr);   // that sweep took the totals, it is no iteration
         if (res.done && !spec) CHK(totals());
         if (res.done || !spec) break;
         loop_end(++queued);

@@ -831,7 +831,7 @@ __device__ __forceinline__ void fluid_nbrs(const NbrLists& L, uint32_t cap, uint
     }
 }
 
-// The same with the list head loaded beforehand (hd = list_head(L, sn, cap, i)).
+// The same with the list head loaded beforehand (list_head, list_head_rest).
 template <uint32_t CAP = kStageMax, class FL, class FG, class Body>
 __device__ __forceinline__ void fluid_nbrs(const NbrLists& L, uint32_t cap, uint32_t b, uint32_t i, uint32_t sn,
                                            const Head& hd, FL&& lds, FG&& glob, Body&& body)
@@ -865,13 +865,6 @@ __device__ __forceinline__ float wave_max(float v)
 {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
-__device__ __forceinline__ uint32_t wave_max_u(uint32_t v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) { const uint32_t w = __shfl_xor(v, o, 64); v = v > w ? v : w; }
     return v;
 }
 

@@ -1205,6 +1205,9 @@ __global__ __launch_bounds__(kBlock) void k_solve_finalize(SolveCtl* ctl, const 
 // the last solve's kappaV increments.  Velocities are read from vel_i and
 // written to vel_o.  The applied k_i starts the particle's total of the step
 // in kvtot (when given).
+// <0, true, true> (bodies) is two registers over the 128 of two blocks per CU and
+// keeps an address in scratch across the loop over 32-bit lists; with the own mass
+// from the constants it fits, but takes 33.5 us instead of 33.1 in the wave tank (260k).
 template <int WS, bool SOL, bool UM>
 __global__ __launch_bounds__(kBlock, UM ? DFSPH_PV_WAVES : 1) void k_div_ws_init(SimConst c, const DevTime* t, uint32_t n,
                                                         const float4* __restrict__ pos,
@@ -1545,8 +1548,11 @@ __global__ void k_update_vel(const DevTime* t, uint32_t n, const float4* acc, fl
 // kws holds the last solve's kappa increments.  No gate (unlike the divergence
 // warm start).  The applied k_i starts the particle's total of the step in
 // ktot (when given).
-// With a uniform mass the stage is the Jacobi sweep's 16-byte records (52 KB, three
-// blocks per CU; 20-byte ones kept two: 203 us for 4.19 M particles, now 173).
+// With a uniform mass the stage is the Jacobi sweep's 16-byte records, 52 KB, which
+// fit three blocks per CU where 20-byte ones fit two.  The plain warm start
+// without bodies keeps to their 80 registers too (4.19 M particles 203 -> 173 us); with
+// bodies or the learned start and the velocity update it takes 81 to 84 and two
+// blocks (held to 80 it spills: wave tank of 260k 20 us, 150k learned 16 to 17, both either way).
 template <int WS, bool APPLY_ACC, bool SOL, bool UM>
 __global__ __launch_bounds__(kBlock) void k_pressure_ws(SimConst c, const DevTime* t, uint32_t n,
                                                         const float4* __restrict__ pos,

@@ -10,8 +10,8 @@
 namespace dfsph {
 
 uint32_t grid_blocks_xcd(uint32_t n);
-uint32_t search_split(uint32_t n);
-uint32_t list_stream(uint32_t n);        // blocks of the search per sweep block
+uint32_t search_split(uint32_t n);       // blocks of the search per sweep block
+uint32_t list_stream(uint32_t n);        // what sweeps over n particles read past the caches (kStreamLists, kStreamIds)
 
 // Kernel timing bound to a dispatch: the next single-kernel sweep launch on
 // this thread (the source, Jacobi, warm-start, XSPH, feature and position
