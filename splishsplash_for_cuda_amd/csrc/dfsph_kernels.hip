@@ -1872,19 +1872,21 @@ uint32_t search_split(uint32_t n)
 }
 
 // What the sweeps over n particles read past the caches (non-temporal loads).
-// A pass reads some 128 bytes a particle, half of them its list, and the passes
-// of a step read the same lists again: up to the 256 MB of the memory-side
-// cache they stay there, and streaming them costs 5 % (1.05 M: Jacobi 50.4 -> 52
-// us).  Beyond, the lists only drive out the records the blocks' sets are gathered
-// from.  Lists streamed, divergence Jacobi: 1.57 M 51.3 -> 52.8 us, 1.84 M 64.2
-// -> 61.5 (but loop end 73.5 -> 75.5), 2.1 M 76.1 -> 68.7, 3.1 M 117 -> 100, 4.2 M
-// 157 -> 137, 6.6 M 234 -> 216.  The sets' ids with them: 2.1 M 68.7 -> 70.7, 3.1 M
-// even, 4.2 M 137 -> 130, 6.6 M 216 -> 210.
+// A pass reads some 128 bytes a particle, the 16-bit lists among them, and the passes
+// of a step read the same again: up to the 256 MB of the memory-side cache
+// it stays there.  Beyond, the lists (read once a pass) drive out the records
+// that the blocks' sets are gathered from; the rest, some 85 bytes, fits longer, and
+// then the sets' ids go the same way.  Both sides, divergence (4 iterations) plus density
+// solve (3), us, at 29 neighbors and walls at spacing 2r (r):
+//   n, M       1.46        1.83        2.12        2.81        3.20        3.63        4.19        5.73
+//   cached     924 (1071) 1185 (1382) 1392 (1636) 1881 (2153) 2146 (2406) 2433 (2772) 2804 (3163) 3747 (4200)
+//   lists      985 (1128) 1195 (1358) 1338 (1508) 1690 (1928) 1956 (2218) 2227 (2560) 2624 (2982) 3606 (4098)
+//   and ids   1006 (1141) 1223 (1376) 1368 (1535) 1723 (1917) 1939 (2157) 2150 (2463) 2483 (2859) 3496 (4025)
 uint32_t list_stream(uint32_t n)
 {
-    constexpr uint32_t kPassBytes = 128u, kCacheBytes = 1u << 28;
+    constexpr uint32_t kPassBytes = 128u, kRestBytes = 85u, kCacheBytes = 1u << 28;
     if (n < kCacheBytes / kPassBytes) return 0u;
-    return n < 2u * (kCacheBytes / kPassBytes) ? kStreamLists : kStreamLists | kStreamIds;
+    return n < kCacheBytes / kRestBytes ? kStreamLists : kStreamLists | kStreamIds;
 }
 
 static thread_local hipEvent_t tl_ev_start = nullptr, tl_ev_stop = nullptr;

@@ -274,3 +274,9 @@ def test_unsorted_search(name):
         f = int(sf[k])
         assert np.array_equal(ids[G[k, :f]], L[i, :f])
         assert np.array_equal(G[k, f:f + int(sb[k])], L[i, f:f + int(sb[k])])
+
+
+@pytest.mark.parametrize("n", [(1 << 28) // 85 - 1, (1 << 28) // 85])
+def test_streamed_ids(n):
+    """The same on both sides of the size from which the ids are streamed too."""
+    test_streamed_lists(n)
