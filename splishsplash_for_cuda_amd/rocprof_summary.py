@@ -62,8 +62,8 @@ def read_counter(path, counter):
 
 
 def min_working(vals, frac=0.5):
-    """Values of working dispatches: velocity sweeps that exit at once (loop
-    already converged) read almost nothing and are left out."""
+    """Values of working dispatches: velocity sweeps that find the loop
+    converged only take the step's totals and are left out."""
     if not vals:
         return vals
     top = max(vals)
@@ -101,8 +101,8 @@ def main():
                     short(row["Name"]), row["Calls"], float(row["AverageNs"]) / 1e3, float(row["MinNs"]) / 1e3,
                     float(row["TotalDurationNs"]) / 1e6, float(row["Percentage"])))
         lines.append("")
-        lines.append("The velocity sweeps (`k_jacobi`) include at most one launch per solve that exits at once "
-                     "(loop already converged); their minimum shows it.")
+        lines.append("The velocity sweeps (`k_jacobi`) include at most one launch per solve that finds the loop "
+                     "converged and takes the step's totals instead; their minimum shows it.")
         lines.append("")
 
     trace_path = os.path.join(d, "trace", "run_kernel_trace.csv")
